@@ -1708,6 +1708,8 @@ static int mat_args(const fdkhip_geom *g, int na, const double *beta, int ia_ski
 	a.dso = g->dso; a.dsd = g->dsd; a.ds = g->ds; a.dt = g->dt;
 	a.offset_source = offset_source;
 	a.scale = scale;
+	a.rdt_h = 1.0 / g->dt;
+	a.rdt_l = fma(-g->dt, a.rdt_h, 1.0) * a.rdt_h;
 	return FDKHIP_OK;
 }
 
@@ -1734,10 +1736,18 @@ static int mat_run(MatArgs &a, const double *beta, const double *source_zs, int 
 {
 	const size_t nxy = (size_t) a.nx * a.ny;
 	std::vector<double4> views = mat_views(beta, source_zs, a.nv, ia_skip);
-	DevBuf dviews, dmask;
+	// the kernel's fast form takes quotients by dt from its reciprocal, within a
+	// range, and pairs of samples from a row
+	bool fast = a.ns >= 2 && fabs(a.dt) > 1e-60 && fabs(a.dt) < 1e60 && fabs(a.dz) < 1e60
+		&& fabs(a.wz) < 1e60;
+	for (const double4 &v : views)
+		fast = fast && fabs(v.z) < 1e60;
+	DevBuf dviews, dmask, dredo;
 	hipError_t e = hipSuccess;
 	if (a.nv > 0)
 		e = hipMalloc(&dviews.p, views.size() * sizeof(double4));
+	if (e == hipSuccess && fast && mat_blocks(a) > 0)
+		e = hipMalloc(&dredo.p, (size_t) mat_blocks(a) * sizeof(int));
 	if (e == hipSuccess && mask_host && nxy > 0)
 		e = hipMalloc(&dmask.p, nxy);
 	if (e != hipSuccess)
@@ -1749,6 +1759,7 @@ static int mat_run(MatArgs &a, const double *beta, const double *source_zs, int 
 		HIP_TRY(hipMemcpyAsync(dmask.p, mask_host, nxy, hipMemcpyHostToDevice, s));
 	a.views = (const double4 *) dviews.p;
 	a.mask = (const uint8_t *) dmask.p;
+	a.redo = (int *) dredo.p;
 	hipEvent_t ev[2] = {nullptr, nullptr};
 	if (kernel_ms) {
 		HIP_TRY(hipEventCreate(&ev[0]));

@@ -90,6 +90,7 @@ struct HelixArgs {
 // cbct_back_mat (fbp/cbct_back.m:142-270): the MATLAB backprojector, all in
 // double as MATLAB holds it.  ws and wt are 1-based (cbct_back.m:185-186).
 constexpr int MAT_ZC = 16;   // slices per lane
+constexpr int MAT_NW = 8;    // most waves (slice chunks) per workgroup
 struct MatArgs {
 	int nx, ny, nz, ns, nt, nv, nzc, kind;   // nv views used, nzc = ceil(nz / MAT_ZC)
 	double dx, dy, dz, wx, wy, wz, ws, wt;
@@ -105,7 +106,12 @@ struct MatArgs {
 	int cone_par;            // views rebinned to cone-parallel geometry
 	double dz_per_rad;       // source height step per radian (cone_par)
 	const double *zscale;    // [nz] per-slice scale, or NULL for `scale`
+	double rdt_h, rdt_l;     // 1 / dt rounded to double, and the rest of it
+	int *redo;               // [mat_blocks] set by the fast form where the other has to
+	                         // do a workgroup again; NULL: the other form alone
 };
+// workgroups of a launch (before redo is set)
+long mat_blocks(const MatArgs &a);
 
 size_t back_lds_bytes(int nw, int vstage, int slot, int fmt);
 // nw consumer waves, zl slices per chunk, zr chunks per wave (interleaved);

@@ -245,3 +245,21 @@ def test_cbct_back_helix_use_mex_0(device, case):
         assert got.dtype == np.float64 and got.shape == (ig.nx, ig.ny, ig.nz)
         assert np.abs(want).max() > 0
         _compare("arc" if (case == "arc" or cone_par) else "flat", got, want)
+
+
+@pytest.mark.parametrize("nz,ns,dt", [(1, 2, 1.3), (16, 7, -1.3), (17, 3, 1.3), (129, 9, 1.3),
+                                      (140, 1, 1.3), (5, 8, 1e-70)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_mat_slice_groups(device, nz, ns, dt, dtype):
+    """Volumes of one slice, of whole and broken 16-slice chunks and of more
+    than one 128-slice workgroup, detectors of one to three columns (the last
+    column's pair of samples lies to its left; one column has no pair), a
+    negative row spacing and one outside the reciprocal quotients' range:
+    bit for bit the restatement, as the same operations are rounded."""
+    g = O.geom((9, 10, nz), (1.1, -1.1, 0.7), (0.25, 0.0, -1.5), 541.0, 949.0, np.inf,
+               ns, 6, (9.0, dt), (0.25, 0.5))
+    rng = np.random.default_rng(nz)
+    proj = rng.standard_normal((ns, 6, 11)).astype(dtype)
+    beta = np.linspace(0, 6, 11)
+    got = _host_call(g, proj, beta, scale=0.3)
+    assert np.array_equal(got, O.back_mat_f64(g, proj, beta, scale=0.3))
