@@ -298,7 +298,7 @@ static void drop_graph(fdkhip_plan *p)
 static bool choose_layout(int nw, int fmt, int maxarea, int vstage_req, int slot_cap,
 	size_t lds_limit, int &vstage_out, int &slot_out)
 {
-	int slot = (std::max(maxarea, 64) + 63) & ~63;
+	int slot = (std::max(maxarea, 64) + 15) & ~15;
 	if (slot_cap > 0)
 		slot = std::max(64, std::min(slot, slot_cap & ~63));
 	const int floor_vs = vstage_req > 0 ? vstage_req : 4;
@@ -306,7 +306,7 @@ static bool choose_layout(int nw, int fmt, int maxarea, int vstage_req, int slot
 	while (vstage > floor_vs && back_lds_bytes(nw, vstage, slot, fmt) > lds_limit)
 		--vstage;
 	while (slot > 64 && back_lds_bytes(nw, vstage, slot, fmt) > lds_limit)
-		slot -= 64;
+		slot -= 16;
 	while (vstage > 1 && back_lds_bytes(nw, vstage, slot, fmt) > lds_limit)
 		--vstage;
 	if (back_lds_bytes(nw, vstage, slot, fmt) > lds_limit)

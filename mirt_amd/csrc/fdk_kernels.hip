@@ -16,13 +16,13 @@
 //   * views go in stages of `vstage` views through two LDS buffers:
 //       setup   -- one lane per (view, column) computes the per-column
 //                  quantities (s bin, weights, slice range, t_bin), packs
-//                  them in a 32-byte record, and a DPP wave reduction gives
+//                  them in a 24-byte record, and a DPP wave reduction gives
 //                  the view's detector footprint over the tile;
 //       stage   -- the footprint of the zero-padded view (the padded copy
 //                  plays fdk_ts_put_view, mex/src/fdk/fdk-orig/fdk,ts,t.c:13-21)
 //                  is copied from HBM into LDS with asynchronous
-//                  global-to-LDS loads (FP32 samples, or FP16/BF16 column
-//                  pairs);
+//                  global-to-LDS loads (FP32 samples), or through registers
+//                  (FP16/BF16 column pairs);
 //       update  -- every consumer lane runs its ZL slices: bilinear
 //                  interpolation from LDS, FP32 accumulation in registers;
 //   * one write per voxel at the end, into the [nz nx ny] image.
@@ -90,13 +90,25 @@ struct ViewGeo {
 	int izb0, izb1;
 };
 
+// Entry of a table that no kernel writes while it is read, at an index that is
+// the same in every lane: through the constant address space, so that it is a
+// scalar load (the compiler takes a vector load where a store of the kernel
+// might alias the table)
+template <typename T>
+__device__ __forceinline__ T table_entry(const T *p, int i)
+{
+	return *(const __attribute__((address_space(4))) T *) (uintptr_t) (p + i);
+}
+typedef float vec2f __attribute__((ext_vector_type(2)));
+typedef int vec2i __attribute__((ext_vector_type(2)));
+
 __device__ __forceinline__ ViewGeo view_geo(const BackArgs &a, int v)
 {
-	const float2 cs = a.trig[v];
+	const vec2f cs = table_entry(reinterpret_cast<const vec2f *>(a.trig), v);
 	ViewGeo vg{cs.x, cs.y, a.g.wz, 0, a.g.nz};
 	if (a.vzs) {
-		vg.wzb = a.g.wz + a.vzs[v] / a.g.dz;
-		const int2 w = a.izb[v];
+		vg.wzb = a.g.wz + table_entry(a.vzs, v) / a.g.dz;
+		const vec2i w = table_entry(reinterpret_cast<const vec2i *>(a.izb), v);
 		vg.izb0 = w.x;
 		vg.izb1 = w.y;
 	}
@@ -146,6 +158,27 @@ __device__ __forceinline__ int column_setup(const GeomF &g, float xx, float yy,
 	return SETUP_ACTIVE;
 }
 
+// atan(x / y) for y > 0, r = 1 / y.  |x| <= y: x r and an odd polynomial, a
+// minimax fit of atan(q) / q in q^2 over [0, 1] made for this (within 1.01 ulp of
+// atan(q) in FP32, 0.30 ulp rms); a wave with a steeper column (more than 45
+// degrees off the central ray) takes the library's atan2f.
+__device__ __forceinline__ float atan_ratio(float x, float y, float r)
+{
+	if (__any(fabsf(x) > y))
+		return atan2f(x, y);
+	const float q = x * r, z = q * q;
+	float p = -0x1.cbc816p-10f;
+	p = fmaf(p, z, 0x1.5f800ap-7f);
+	p = fmaf(p, z, -0x1.f8b3c6p-6f);
+	p = fmaf(p, z, 0x1.d7777ap-5f);
+	p = fmaf(p, z, -0x1.572282p-4f);
+	p = fmaf(p, z, 0x1.c02f82p-4f);
+	p = fmaf(p, z, -0x1.24159ap-3f);
+	p = fmaf(p, z, 0x1.999082p-3f);
+	p = fmaf(p, z, -0x1.555534p-2f);
+	return fmaf(q, p * z, q);
+}
+
 // Per-column, per-view quantities for the FP16/BF16 paths, which are held to
 // the FP64 result rather than to the reference's bits: reciprocals instead
 // of divisions, float atan2 for the arc detector, FMA.  iz_min/iz_max are
@@ -158,7 +191,7 @@ __device__ __forceinline__ int column_setup_fast(const GeomF &g, float xx, float
 	const float ybetas = g.dso - fmaf(-xx, sinb, yy * cosb);
 	const float rb = __builtin_amdgcn_rcpf(ybetas);
 	const float mag = (g.kind == KIND_PAR) ? 1.f : g.dsd * rb;
-	const float ss = (g.kind == KIND_ARC) ? g.dsd * atan2f(xbeta, ybetas) : mag * xbeta;
+	const float ss = (g.kind == KIND_ARC) ? g.dsd * atan_ratio(xbeta, ybetas, rb) : mag * xbeta;
 	const float ss_bin = fmaf(ss, g.inv_ds, g.ws);
 	if (!(ss_bin >= -1.f && ss_bin < (float) g.ns))   // also rejects NaN
 		return SETUP_OUT;
@@ -355,31 +388,30 @@ __device__ __forceinline__ bool col_range(const GeomF &g, float xx, float yy, co
 	return true;
 }
 
-// Wave-wide reductions (wave64, every lane active) with DPP: quad swaps,
-// row half-mirror and mirror give each row of 16 its result, row_bcast:15
-// and :31 carry it across rows; lane 63 holds the wave's result.  The
-// operation's identity as the DPP "old" value (what lanes outside the row
-// mask receive) lets the compiler fold each step into one v_min/v_max_dpp.
-template <bool MAX>
-__device__ __forceinline__ int wave_reduce(int v)
+// Wave-wide minima (wave64, every lane active) of N values at once with DPP:
+// quad swaps, row half-mirror and mirror give each row of 16 its result,
+// row_bcast:15 and :31 carry it across rows; lane 63 holds the wave's result.
+// The operation's identity as the DPP "old" value (what lanes outside the row
+// mask receive) lets the compiler fold each step into one v_min_dpp; several
+// values in step fill the wait states between a result and its DPP use.
+// A maximum is a minimum of the complements: max(x) = ~min(~x).
+template <int N>
+__device__ __forceinline__ void wave_min_n(int (&v)[N])
 {
-	auto op = [](int a, int b) { return MAX ? max(a, b) : min(a, b); };
-	constexpr int id = MAX ? (int) 0x80000000 : 0x7fffffff;
-	v = op(v, __builtin_amdgcn_update_dpp(id, v, 0xb1, 0xf, 0xf, false));   // quad_perm 1,0,3,2
-	v = op(v, __builtin_amdgcn_update_dpp(id, v, 0x4e, 0xf, 0xf, false));   // quad_perm 2,3,0,1
-	v = op(v, __builtin_amdgcn_update_dpp(id, v, 0x141, 0xf, 0xf, false));  // row_half_mirror
-	v = op(v, __builtin_amdgcn_update_dpp(id, v, 0x140, 0xf, 0xf, false));  // row_mirror
-	v = op(v, __builtin_amdgcn_update_dpp(id, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
-	v = op(v, __builtin_amdgcn_update_dpp(id, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
-	return __builtin_amdgcn_readlane(v, 63);
-}
-__device__ __forceinline__ int wave_min(int v)
-{
-	return wave_reduce<false>(v);
-}
-__device__ __forceinline__ int wave_max(int v)
-{
-	return wave_reduce<true>(v);
+	constexpr int id = 0x7fffffff;
+#define FDK_DPP_STEP(CTRL, ROWS)                                                           \
+	_Pragma("unroll") for (int i = 0; i < N; ++i)                                          \
+		v[i] = min(v[i], __builtin_amdgcn_update_dpp(id, v[i], CTRL, ROWS, 0xf, false));
+	FDK_DPP_STEP(0xb1, 0xf)    // quad_perm 1,0,3,2
+	FDK_DPP_STEP(0x4e, 0xf)    // quad_perm 2,3,0,1
+	FDK_DPP_STEP(0x141, 0xf)   // row_half_mirror
+	FDK_DPP_STEP(0x140, 0xf)   // row_mirror
+	FDK_DPP_STEP(0x142, 0xa)   // row_bcast:15
+	FDK_DPP_STEP(0x143, 0xc)   // row_bcast:31
+#undef FDK_DPP_STEP
+#pragma unroll
+	for (int i = 0; i < N; ++i)
+		v[i] = __builtin_amdgcn_readlane(v[i], 63);
 }
 
 // Logical block index with consecutive indices on the same XCD: the hardware
@@ -403,36 +435,39 @@ extern __shared__ float fdk_lds[];
 // after them two zero words that DIRECT lanes without work in a view read.
 //   slots [vstage][slot]        staged footprints: FP32 samples (walk modes),
 //                               16-bit column pairs (DIRECT)
-//   P     [vstage][64][8]       per (view, column) record, two 16-byte halves
-//                               read with one ds_read_b128 each:
-//     walk:   P0 = {cb, wl, wr, w2}      P1 = {t_inc, zlo | zhi << 16, is, t_last}
-//     DIRECT: P0 = {cb, wl, wr, U0}      P1 = {t_inc, zlo | zhi << 16, u_hi, 0}
-//             (DIRECT wl, wr: FP32 horizontal weights times w2 times the
-//             view scale)
-//           cb: LDS word, relative to the stage buffer, of the lane's left
-//               column at row 1 (walk) / padded row 0 (DIRECT); for views
-//               gathered from HBM: is
+//   P     [vstage][64][4]       per (view, column) record, read with one
+//                               ds_read_b128:
+//     walk:   {cb, wl, wr, w2}
+//     DIRECT: {cb, wl, wr, U0} (wl, wr: FP32 horizontal weights times w2
+//             times the view scale)
+//   Q     [vstage][64][2]       the rest of it: walk {t_inc, zlo | zhi << 16},
+//                               DIRECT {t_inc, u_hi}
+//     cb: LDS word, relative to the stage buffer, of the lane's left column at
+//         row 1 (walk) / padded row 0 (DIRECT); for views gathered from HBM: is
+//         (DIRECT lanes without work: NO_COLUMN)
 //   T     [vstage][NW][64]      walk only: t_bin at each consumer wave's first
 //                               active slice (DIRECT evaluates it from U0)
 //   vinfo [vstage][4]           mode | zlo << 2 | zhi << 12: the union of the
 //                               tile's slice ranges relative to the z-group
-//                               (at most 256 slices), and ilo | ihi << 10:
-//                               their intersection (walk modes with several
-//                               chunks per wave; with one: s_lo, t_lo),
+//                               (at most 256 slices), and ilo | ihi << 10: the
+//                               slices all its columns cover (walk modes with
+//                               one chunk per wave: s_lo, t_lo),
 //                               tw, (mode << 16) | staged columns
 template <int NW, bool TTAB>
 struct Lds {
-	int P, T, vinfo, total, zero;
+	int P, Q, T, vinfo, total, zero;
 	__device__ __forceinline__ Lds(int vstage, int slot)
 	{
 		P = vstage * slot;
-		T = P + vstage * 64 * 8;
+		Q = P + vstage * 64 * 4;
+		T = Q + vstage * 64 * 2;
 		vinfo = T + (TTAB ? vstage * NW * 64 : 0);
 		total = vinfo + vstage * 4;
 		zero = 2 * total;
 	}
 };
 
+constexpr int NO_COLUMN = -3;   // pairs (-3, -2) and further left read zeros
 enum { MODE_LDS = 0, MODE_GLOBAL = 1, MODE_NONE = 2 };
 
 // Detector footprint of one view over the tile and z-group in padded
@@ -444,15 +479,12 @@ struct Footprint {
 	int s_lo, s_hi, t_lo, t_hi;
 };
 
-template <bool DIRECT>
 __device__ __forceinline__ Footprint view_footprint(const GeomF &g, bool act, const ColRange &cr)
 {
-	Footprint f;
-	f.s_lo = max(wave_min(act ? cr.c.is + 1 : 0x7fffffff), 0);
-	f.s_hi = min(wave_max(act ? cr.c.is + 2 : (int) 0x80000000), g.ns + 1);
-	f.t_lo = max(wave_min(act ? cr.row_lo : 0x7fffffff), 0);
-	f.t_hi = min(wave_max(act ? cr.row_hi : (int) 0x80000000), g.nt + 2);
-	return f;
+	int m[4] = {act ? cr.c.is + 1 : 0x7fffffff, act ? ~(cr.c.is + 2) : 0x7fffffff,
+		act ? cr.row_lo : 0x7fffffff, act ? ~cr.row_hi : 0x7fffffff};
+	wave_min_n(m);
+	return Footprint{max(m[0], 0), min(~m[1], g.ns + 1), max(m[2], 0), min(~m[3], g.nt + 2)};
 }
 
 // Asynchronous copy of one FP32 sample per lane from HBM into the LDS word
@@ -465,54 +497,86 @@ __device__ __forceinline__ void stage_word(const char *src, float *ldst)
 	__builtin_amdgcn_global_load_lds(g, l, 4, 0, 0);
 }
 
+// LDS byte address of word `w` of the kernel's LDS array
+__device__ __forceinline__ uint32_t lds_byte(int w)
+{
+	return (uint32_t) (uintptr_t) (__attribute__((address_space(3))) float *) (fdk_lds + w);
+}
+
+// N column pairs of a DIRECT footprint, at one detector row per lane: the
+// samples of N columns from `col` (the byte address of a column's first sample,
+// the same in every lane) in flight together, then the words to LDS.  prev is
+// the column before, and afterwards the last one.
+template <int N>
+__device__ __forceinline__ void stage_columns(const char *&col, uint32_t colbytes, uint32_t row,
+	uint32_t &prev, uint32_t &dst, uint32_t dstbytes)
+{
+	uint32_t cur[N];
+#pragma unroll
+	for (int q = 0; q < N; ++q)
+		cur[q] = *(const uint16_t *) (col + (size_t) q * colbytes + row);
+#pragma unroll
+	for (int q = 0; q < N; ++q) {
+		*(__attribute__((address_space(3))) uint32_t *) (uintptr_t) dst = prev | (cur[q] << 16);
+		prev = cur[q];
+		dst += dstbytes;
+	}
+	col += (size_t) N * colbytes;
+}
+
+// (clinical_arc FP16, 984 views of 888 x 64 to 512^2 x 256: with this staging,
+// the arc's own arctangent and the 24-byte records 7.7 ms; 8.6 ms with clamped
+// 64-bit column addresses and a lane mask per column.)
+//
 // DIRECT staging of one view's footprint: slot word (k, r), k in [0, sw),
 // r in [0, tw), holds the padded samples (s_lo + k, t_lo + r) in its low and
 // (s_lo + k + 1, t_lo + r) in its high half, read straight from the caller's
 // [ns][nt] 16-bit view and zero outside [1, ns] x [1, nt] (the zero border
 // that fdk_ts_put_view gives each view, fdk,ts,t.c:13-21).  Lane = detector
 // row: the wave walks the columns keeping the previous column's sample, with
-// sixteen 2-byte loads in flight (64 consecutive samples of a column per
-// load, one 128-byte line).  Each sample is read from HBM once per footprint.
-// Columns are tw words apart (the caller makes tw odd, so that lanes reading
-// the same row of neighbouring columns fall in different LDS banks).
+// up to sixteen 2-byte loads in flight (64 consecutive samples of a column per
+// load, one 128-byte line) from scalar column addresses.  Each sample is read
+// from HBM once per footprint.  Columns are tw words apart (the caller makes
+// tw odd, so that lanes reading the same row of neighbouring columns fall in
+// different LDS banks).
 __device__ __forceinline__ void stage_pairs(const uint16_t *view, const GeomF &g,
 	const Footprint &f, int sw, int tw, int slot, int lane)
 {
-	// zero rows of the footprint: padded rows 0, nt + 1 and nt + 2
-	for (int q = 0; q < 3; ++q) {
-		const int zr = (q == 0) ? 0 : g.nt + q;
-		if (zr < f.t_lo || zr > f.t_hi)
-			continue;
+	// zero rows of the footprint: below padded row 1 and above row nt
+	const int rows = f.t_hi - f.t_lo + 1;
+	const int zlo = min(max(1 - f.t_lo, 0), rows), zhi = min(max(f.t_hi - g.nt, 0), rows);
+	for (int q = 0; q < zlo + zhi; ++q) {
+		const int r = q < zlo ? q : rows - 1 - (q - zlo);
 		for (int k = lane; k < sw; k += 64)
-			fdk_lds[slot + k * tw + (zr - f.t_lo)] = 0.f;
+			fdk_lds[slot + k * tw + r] = 0.f;
 	}
+	const uint32_t colbytes = 2u * (uint32_t) g.nt, dstbytes = 4u * (uint32_t) tw;
+	const char *first = (const char *) view + (size_t) f.s_lo * colbytes;   // sample column s_lo
 	const int ra = max(f.t_lo, 1), rb = min(f.t_hi, g.nt);   // detector rows
+	const int n = sw - (f.s_hi > g.ns ? 1 : 0);   // pairs whose right column is on the detector
 	for (int r0 = ra; r0 <= rb; r0 += 64) {
 		const int r = r0 + lane;
-		const bool rv = r <= rb;
-		const int srow = (rv ? r : rb) - 1;    // sample row (a valid one past the end)
-		const int lw = slot + (r - f.t_lo);
+		if (r > rb)
+			continue;
+		const uint32_t row = 2u * (uint32_t) (r - 1);
+		uint32_t dst = lds_byte(slot + (r - f.t_lo));
 		uint32_t prev = 0u;                    // padded column s_lo (0: the zero pad)
 		if (f.s_lo >= 1)
-			prev = view[(long) (f.s_lo - 1) * g.nt + srow];
-		for (int k0 = 0; k0 < sw; k0 += 16) {
-			uint32_t cur[16];
-#pragma unroll
-			for (int q = 0; q < 16; ++q) {
-				// padded column s_lo + k0 + q + 1 is sample column s_lo + k0 + q;
-				// clamped so that the loads past the footprint stay in the view
-				const int sc = min(f.s_lo + k0 + q, g.ns - 1);
-				cur[q] = view[(long) sc * g.nt + srow];
-			}
-#pragma unroll
-			for (int q = 0; q < 16; ++q) {
-				const int k = k0 + q;
-				const uint32_t hi = (f.s_lo + k + 1 <= g.ns) ? cur[q] : 0u;
-				if (k < sw && rv)
-					fdk_lds[lw + k * tw] = __uint_as_float(prev | (hi << 16));
-				prev = hi;
-			}
-		}
+			prev = *(const uint16_t *) (first - colbytes + row);
+		const char *col = first;
+		int k = n;
+		for (; k >= 16; k -= 16)
+			stage_columns<16>(col, colbytes, row, prev, dst, dstbytes);
+		if (k & 8)
+			stage_columns<8>(col, colbytes, row, prev, dst, dstbytes);
+		if (k & 4)
+			stage_columns<4>(col, colbytes, row, prev, dst, dstbytes);
+		if (k & 2)
+			stage_columns<2>(col, colbytes, row, prev, dst, dstbytes);
+		if (k & 1)
+			stage_columns<1>(col, colbytes, row, prev, dst, dstbytes);
+		if (n < sw)                            // column ns + 1: the zero pad
+			*(__attribute__((address_space(3))) uint32_t *) (uintptr_t) dst = prev;
 	}
 }
 
@@ -536,10 +600,11 @@ __device__ __forceinline__ void produce(const BackArgs &a, int bo,
 		// col_range, and its record must still describe an empty range
 		ColRange cr{};
 		float Tk[NW] = {};
+		const ViewGeo vg = view_geo(a, v);
 		const bool act = colvalid
-			&& col_range<NW, ZL, DIRECT>(g, xx, yy, view_geo(a, v), zg0, zg1, cr, Tk);
+			&& col_range<NW, ZL, DIRECT>(g, xx, yy, vg, zg0, zg1, cr, Tk);
 		const ColSetup &c = cr.c;
-		const Footprint f = view_footprint<DIRECT>(g, act, cr);
+		const Footprint f = view_footprint(g, act, cr);
 		int mode = MODE_NONE, tw = 0, sw = 0;
 		if (f.s_lo <= f.s_hi && f.t_lo <= f.t_hi) {
 			// DIRECT: an odd column stride (bank spread, stage_pairs)
@@ -547,19 +612,18 @@ __device__ __forceinline__ void produce(const BackArgs &a, int bo,
 			sw = f.s_hi - f.s_lo + (DIRECT ? 0 : 1);     // staged columns (DIRECT: pairs)
 			mode = ((long) sw * tw <= a.slot) ? MODE_LDS : MODE_GLOBAL;
 		}
-		const int is_st = act ? c.is : 0;
-		const int zhi_st = act ? cr.zhi : cr.zlo;
-		float4 *P4 = reinterpret_cast<float4 *>(fdk_lds + bo + L.P) + (vv * 64 + lane) * 2;
+		float4 *P4 = reinterpret_cast<float4 *>(fdk_lds + bo + L.P) + vv * 64 + lane;
 		if constexpr (DIRECT) {
 			// LDS word of padded row 0 in the lane's column pair; lanes without
 			// work in this view read the two zero words with zero weights
-			const int cb = !act ? L.zero - bo
-				: (mode == MODE_LDS ? vv * a.slot + (c.is + 1 - f.s_lo) * tw - f.t_lo : c.is);
-			const float w2s = act ? c.w2 * a.scale[v] : 0.f;
-			P4[0] = make_float4(__int_as_float(cb), act ? w2s * c.wl : 0.f,
+			const int cb = mode == MODE_LDS
+				? (act ? vv * a.slot + (c.is + 1 - f.s_lo) * tw - f.t_lo : L.zero - bo)
+				: (act ? c.is : NO_COLUMN);
+			const float w2s = act ? c.w2 * table_entry(a.scale, v) : 0.f;
+			*P4 = make_float4(__int_as_float(cb), act ? w2s * c.wl : 0.f,
 				act ? w2s * c.wr : 0.f, act ? Tk[0] : 0.f);
-			P4[1] = make_float4(act ? c.t_inc : 0.f,
-				__int_as_float(act ? cr.zlo | (zhi_st << 16) : 0), act ? cr.u_hi : 0.f, 0.f);
+			reinterpret_cast<float2 *>(fdk_lds + bo + L.Q)[vv * 64 + lane] =
+				make_float2(act ? c.t_inc : 0.f, act ? cr.u_hi : 0.f);
 		} else {
 			// LDS word of row 1, t = 0 in the lane's left column
 			const int cb = act ? vv * a.slot + (c.is + 1 - f.s_lo) * tw + 1 - f.t_lo : 0;
@@ -569,10 +633,10 @@ __device__ __forceinline__ void produce(const BackArgs &a, int bo,
 				wl = w2 * wl;
 				wr = w2 * wr;
 			}
-			P4[0] = make_float4(__int_as_float(mode == MODE_LDS ? cb : is_st), wl, wr, w2);
-			P4[1] = make_float4(act ? c.t_inc : 0.f,
-				__int_as_float(act ? cr.zlo | (zhi_st << 16) : 0), __int_as_float(is_st),
-				act ? cr.last : 0.f);
+			*P4 = make_float4(__int_as_float(mode == MODE_LDS ? cb : act ? c.is : 0), wl, wr, w2);
+			reinterpret_cast<float2 *>(fdk_lds + bo + L.Q)[vv * 64 + lane] =
+				make_float2(act ? c.t_inc : 0.f,
+					__int_as_float(act ? cr.zlo | (cr.zhi << 16) : 0));
 			// t_bin at each chunk's first active slice; chunks the lane's range
 			// misses get t_first, so that their (discarded) reads stay inside
 			// the staged footprint
@@ -591,14 +655,16 @@ __device__ __forceinline__ void produce(const BackArgs &a, int bo,
 		// with none active the view's mode is MODE_NONE and no range is read.
 		int zrange = 0, zboth = 0;
 		if constexpr (DIRECT || R > 1) {
-			const int zl = wave_min(act ? cr.zlo - zg0 : 0x7fffffff);
-			const int zh = wave_max(act ? cr.zhi - zg0 : (int) 0x80000000);
-			zrange = (mode == MODE_NONE) ? 0 : (zl << 2) | (zh << 12);
+			int m[DIRECT ? 2 : 4] = {act ? cr.zlo - zg0 : 0x7fffffff,
+				act ? ~(cr.zhi - zg0) : 0x7fffffff};
 			if constexpr (!DIRECT) {
-				const int il = min(wave_max(act ? cr.zlo - zg0 : 1023), 1023);
-				const int ih = max(wave_min(act ? cr.zhi - zg0 : 0), 0);
-				zboth = il | (ih << 10);
+				m[2] = act ? ~(cr.zlo - zg0) : ~1023;
+				m[3] = act ? cr.zhi - zg0 : 0;
 			}
+			wave_min_n(m);
+			zrange = (mode == MODE_NONE) ? 0 : (m[0] << 2) | (~m[1] << 12);
+			if constexpr (!DIRECT)
+				zboth = min(~m[2], 1023) | (max(m[3], 0) << 10);
 		}
 		if (lane == 0) {
 			int *vi = reinterpret_cast<int *>(fdk_lds) + bo + L.vinfo + vv * 4;
@@ -710,12 +776,11 @@ __device__ __forceinline__ float pair_hi(uint32_t w)
 		return __uint_as_float(w & 0xffff0000u);
 }
 
-// Bilinear interpolation of FP16/BF16 samples with FP32 weights, added to
-// acc in FP32: a0, b0 on the lower row, a1, b1 on the upper one, wl, wr the
-// horizontal weights (w2 and the view scale folded in), wu the vertical one.
-// -q1 and q2 - q1 come from two chains of two FMAs (for FP16 each one
-// v_fma_mix_f32, which widens the 16-bit sample inside the instruction),
-// then acc + q1 + wu * (q2 - q1).
+// Bilinear interpolation with FP32 weights, added to acc: a0, b0 on the lower
+// row, a1, b1 on the upper one, wl, wr the horizontal weights (w2 and the view
+// scale folded in), wu the vertical one.  -q1 and q2 - q1 come from two chains
+// of two FMAs (for FP16 samples each one v_fma_mix_f32, which widens the
+// sample inside the instruction), then acc + q1 + wu * (q2 - q1).
 __device__ __forceinline__ float bilerp_d(float acc, float a0, float b0, float a1, float b1,
 	float wl, float wr, float wu)
 {
@@ -765,28 +830,31 @@ __device__ __forceinline__ void consume_walk(const BackArgs &a, int bo,
 {
 	constexpr int NC = NW * R;
 	const GeomF &g = a.g;
-	const float4 *P4 = reinterpret_cast<const float4 *>(fdk_lds + bo + L.P) + lane * 2;
+	const float4 *P4 = reinterpret_cast<const float4 *>(fdk_lds + bo + L.P) + lane;
+	const float2 *Q2 = reinterpret_cast<const float2 *>(fdk_lds + bo + L.Q) + lane;
 	const float *Tw = fdk_lds + bo + L.T + wave * 64 + lane;
 	// R > 1: the view's four info words; R = 1: tw and mode (the last two)
 	using Info = std::conditional_t<(R > 1), int4, int2>;
 	constexpr int IW = R > 1 ? 1 : 2;   // Info entries per view
 	const Info *VI = reinterpret_cast<const Info *>(fdk_lds + bo + L.vinfo + (R > 1 ? 0 : 2));
-	float4 np0 = P4[0], np1 = P4[1];
+	float4 np0 = P4[0];
+	float2 np1 = Q2[0];
 	float nts[R];
 #pragma unroll
 	for (int r = 0; r < R; ++r)
 		nts[r] = Tw[r * NW * 64];
 	Info nvi = VI[0];
 	for (int vv = 0; vv < nv; ++vv) {
-		const float4 p0 = np0, p1 = np1;
+		const float4 p0 = np0;
+		const float2 p1 = np1;
 		const Info vi = nvi;
 		float ts[R];               // t_bin at the lane's first active slice of each chunk
 #pragma unroll
 		for (int r = 0; r < R; ++r)
 			ts[r] = nts[r];
 		if (vv + 1 < nv) {
-			np0 = P4[(vv + 1) * 128];
-			np1 = P4[(vv + 1) * 128 + 1];
+			np0 = P4[(vv + 1) * 64];
+			np1 = Q2[(vv + 1) * 64];
 #pragma unroll
 			for (int r = 0; r < R; ++r)
 				nts[r] = Tw[((vv + 1) * NC + r * NW) * 64];
@@ -918,8 +986,8 @@ __device__ __forceinline__ int2 view_window(const BackArgs &a, int v)
 {
 	if (!WINDOW)
 		return make_int2((int) 0x80000000, 0x7fffffff);
-	const int2 w = a.izb[v];
-	return make_int2(__builtin_amdgcn_readfirstlane(w.x), __builtin_amdgcn_readfirstlane(w.y));
+	const vec2i w = table_entry(reinterpret_cast<const vec2i *>(a.izb), v);
+	return make_int2(w.x, w.y);
 }
 
 // Consumer side of DIRECT (FP16/BF16 storage): the views staged in LDS
@@ -927,16 +995,17 @@ __device__ __forceinline__ int2 view_window(const BackArgs &a, int v)
 // changes the FP32 summation order -- any view whose footprint exceeded the
 // slot, gathered from HBM.  Keeping the two apart keeps one code path over
 // the accumulators in the main loop, so they stay in place in registers.
-// Every slice of a chunk a wave works on inside the view's slice window is
+// Every slice of a group a wave works on inside the view's slice window is
 // computed with u clamped to [0, u_hi] (ColRange): slices outside a lane's
 // range read zero rows with vertical weight 0, and lanes without work read
-// the zero words.  WINDOW (a helical plan): the view's slice window is the
-// same for every lane; groups of 8 slices that it cuts are added in a
-// second pass over the stage's views, with a select on the window, so that
-// the main loop keeps one code path over the accumulators (and they stay in
-// place in registers).  The slices outside the window
-// are not on the clamp's zero rows when the window, not the cone, ends a
-// lane's range, so they must not be added.
+// the zero words.  (A scalar branch past the clamps where all lanes cover the
+// group costs more than the clamps: clinical_arc FP16 8.6 ms against 8.05.)
+// WINDOW (a helical plan): the view's slice window is the same for every
+// lane; groups of 8 slices that it cuts are added in a second pass over the
+// stage's views, with a select on the window, so that the main loop keeps
+// one code path over the accumulators (and they stay in place in registers).
+// The slices outside the window are not on the clamp's zero rows when the
+// window, not the cone, ends a lane's range, so they must not be added.
 // The R chunks of consumer wave `wave` (of NCW) are chunks wave + r NCW of the
 // z-group, ZL slices each, with accumulators accs[r]; one pass over the
 // stage's views adds all of them (each view's record and window read once).
@@ -946,7 +1015,8 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 	float (&accs)[R][ZL])
 {
 	const GeomF &g = a.g;
-	const float4 *P4 = reinterpret_cast<const float4 *>(fdk_lds + bo + L.P) + lane * 2;
+	const float4 *P4 = reinterpret_cast<const float4 *>(fdk_lds + bo + L.P) + lane;
+	const float2 *Q2 = reinterpret_cast<const float2 *>(fdk_lds + bo + L.Q) + lane;
 	const int2 *VI = reinterpret_cast<const int2 *>(fdk_lds + bo + L.vinfo + 2);
 	const int *ZR = reinterpret_cast<const int *>(fdk_lds + bo + L.vinfo);
 	// relative to the z-group: chunk r starts at slice zoff(r)
@@ -968,8 +1038,6 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 			continue;
 		// the union of the tile's slice ranges (scalar): a group inside it
 		// where some lanes have no slices adds exactly 0 for those lanes
-		// (their u is clamped onto zero rows, or the group is one the view's
-		// window cuts, added with a select below)
 		const int ulo = (zr >> 2) & 1023, uhi = (zr >> 12) & 1023;
 		bool meets = false;
 #pragma unroll
@@ -977,11 +1045,11 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 			meets = meets || (ulo < zoff(r) + ZL && uhi > zoff(r));
 		if (!meets)
 			continue;                  // no lane of this wave meets the view
-		const float4 p0 = P4[vv * 128], p1 = P4[vv * 128 + 1];
+		const float4 p0 = P4[vv * 64];
 		const int c1 = bo + __float_as_int(p0.x);
 		const float wl = p0.y, wr = p0.z;
-		const float ti = p1.x;
-		const float uh = p1.z;
+		const float2 q2 = Q2[vv * 64];
+		const float ti = q2.x, uh = q2.y;
 		const int2 wa = view_window<WINDOW>(a, v0 + vv);
 #pragma unroll
 		for (int r = 0; r < R; ++r) {
@@ -992,50 +1060,43 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 				continue;
 			const float t0 = fmaf((float) zoff(r), ti, p0.w);   // u at the chunk's first slice
 			const int2 w = window(wa, r);
+			// halves of 4 slices; on helical plans groups of 8 (finer tests cost
+			// more than they save where windows cut groups)
+			constexpr int HS = WINDOW ? 8 : 4;
 #pragma unroll
-			for (int g0 = 0; g0 < ZL; g0 += 8) {
-				// groups of 8 slices outside the union are skipped; groups the
-				// view's window cuts (a helix) are left to the pass below
-				if (g0 >= w.y || g0 + 8 <= w.x || g0 >= jhi || g0 + 8 <= jlo)
+			for (int h0 = 0; h0 < ZL; h0 += HS) {
+				// groups outside the union are skipped; groups the view's window
+				// cuts (a helix) are left to the pass below
+				if (h0 >= jhi || h0 + HS <= jlo || h0 >= w.y || h0 + HS <= w.x)
 					continue;
-				if (g0 < w.x || g0 + 8 > w.y) {
+				if (WINDOW && (h0 < w.x || h0 + HS > w.y)) {
 					cut_views = true;
 					continue;
 				}
-				// axial: halves of 4 slices outside the union skipped as well
-				// (finer tests cost more than they save where windows cut groups)
-				constexpr int HS = WINDOW ? 8 : 4;
+				if constexpr (!WINDOW) {
+					// the half's four LDS reads first, then its arithmetic
+					// (a helical plan's 8-slice groups would need the
+					// registers of eight reads in flight)
+					uint32_t w0[HS], w1[HS];
+					float wu[HS];
 #pragma unroll
-				for (int h0 = g0; h0 < g0 + 8; h0 += HS) {
-					if (h0 + HS <= jlo || h0 >= jhi)
-						continue;
-					if constexpr (!WINDOW) {
-						// the half's four LDS reads first, then its arithmetic
-						// (a helical plan's 8-slice groups would need the
-						// registers of eight reads in flight)
-						uint32_t w0[HS], w1[HS];
-						float wu[HS];
+					for (int k = 0; k < HS; ++k) {
+						const float u = __builtin_amdgcn_fmed3f(fmaf((float) (h0 + k), ti, t0),
+							0.f, uh);
+						const int iu = (int) u;
+						wu[k] = __builtin_amdgcn_fractf(u);
+						w0[k] = __float_as_uint(fdk_lds[c1 + iu]);
+						w1[k] = __float_as_uint(fdk_lds[c1 + iu + 1]);
+					}
 #pragma unroll
-						for (int k = 0; k < HS; ++k) {
-							const float u = __builtin_amdgcn_fmed3f(
-								fmaf((float) (h0 + k), ti, t0), 0.f, uh);
-							const int iu = (int) u;
-							wu[k] = __builtin_amdgcn_fractf(u);
-							w0[k] = __float_as_uint(fdk_lds[c1 + iu]);
-							w1[k] = __float_as_uint(fdk_lds[c1 + iu + 1]);
-						}
+					for (int k = 0; k < HS; ++k)
+						acc[h0 + k] = bilerp_d(acc[h0 + k], pair_lo<FMT>(w0[k]), pair_hi<FMT>(w0[k]),
+							pair_lo<FMT>(w1[k]), pair_hi<FMT>(w1[k]), wl, wr, wu[k]);
+				} else {
 #pragma unroll
-						for (int k = 0; k < HS; ++k)
-							acc[h0 + k] = bilerp_d(acc[h0 + k], pair_lo<FMT>(w0[k]),
-								pair_hi<FMT>(w0[k]), pair_lo<FMT>(w1[k]),
-								pair_hi<FMT>(w1[k]), wl, wr, wu[k]);
-					} else {
-#pragma unroll
-						for (int j = h0; j < h0 + HS; ++j) {
-							const float u = __builtin_amdgcn_fmed3f(fmaf((float) j, ti, t0),
-								0.f, uh);
-							acc[j] = slice_update_d<FMT>(acc[j], u, c1, wl, wr);
-						}
+					for (int j = h0; j < h0 + HS; ++j) {
+						const float u = __builtin_amdgcn_fmed3f(fmaf((float) j, ti, t0), 0.f, uh);
+						acc[j] = slice_update_d<FMT>(acc[j], u, c1, wl, wr);
 					}
 				}
 			}
@@ -1058,11 +1119,11 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 			if (!cut)
 				continue;
 			const int ulo = (zr >> 2) & 1023, uhi = (zr >> 12) & 1023;
-			const float4 p0 = P4[vv * 128], p1 = P4[vv * 128 + 1];
+			const float4 p0 = P4[vv * 64];
 			const int c1 = bo + __float_as_int(p0.x);
 			const float wl = p0.y, wr = p0.z;
-			const float ti = p1.x;
-			const float uh = p1.z;
+			const float2 q2 = Q2[vv * 64];
+		const float ti = q2.x, uh = q2.y;
 #pragma unroll
 			for (int r = 0; r < R; ++r) {
 				float (&acc)[ZL] = accs[r];
@@ -1090,30 +1151,27 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 	if (!hbm_views)
 		return;
 	// views whose footprint exceeded the LDS slot: gather from the caller's
-	// views, zero outside the detector; lanes without slices in a view read
+	// views, zero outside the detector; lanes without work in a view read
 	// columns left of the detector (zeros)
 	for (int vv = 0; vv < nv; ++vv) {
 		const int2 vi = VI[vv * 2];
 		if ((__builtin_amdgcn_readfirstlane(vi.y) >> 16) != MODE_GLOBAL)
 			continue;
-		const float4 p0 = P4[vv * 128], p1 = P4[vv * 128 + 1];
-		const int zlohi = __float_as_int(p1.y);
-		const int zlo = zlohi & 0xffff, zhi = (int) ((unsigned) zlohi >> 16);
+		const int zr = __builtin_amdgcn_readfirstlane(ZR[vv * 4]);
+		const int ulo = (zr >> 2) & 1023, uhi = (zr >> 12) & 1023;
+		const float4 p0 = P4[vv * 64];
 		const float wl = p0.y, wr = p0.z;
-		const float ti = p1.x;
-		const float uh = p1.z;
+		const float2 q2 = Q2[vv * 64];
+		const float ti = q2.x, uh = q2.y;
+		const int is = __float_as_int(p0.x);   // the record holds is
 		const uint16_t *pv = static_cast<const uint16_t *>(a.proj)
 			+ (size_t) (v0 + vv) * g.ns * g.nt;
 		const int2 wa = view_window<WINDOW>(a, v0 + vv);
 #pragma unroll
 		for (int r = 0; r < R; ++r) {
 			float (&acc)[ZL] = accs[r];
-			const int zc = zg0 + zoff(r);
-			const int jlo = max(zlo - zc, 0);
-			const int jhi = min(zhi - zc, ZL);
-			if (!__any(jlo < jhi))
+			if (ulo >= zoff(r) + ZL || uhi <= zoff(r))
 				continue;
-			const int is = (jlo < jhi) ? __float_as_int(p0.x) : -3;   // the record holds is
 			const float t0 = fmaf((float) zoff(r), ti, p0.w);
 			const int2 w = window(wa, r);
 #pragma unroll
@@ -1345,7 +1403,7 @@ survey_kernel(const BackArgs a)
 		float Tk[NW];
 		const bool act = colvalid
 			&& col_range<NW, ZL, DIRECT>(g, xx, yy, vg, zg0, zg1, cr, Tk);
-		const Footprint f = view_footprint<DIRECT>(g, act, cr);
+		const Footprint f = view_footprint(g, act, cr);
 		if (f.s_lo <= f.s_hi && f.t_lo <= f.t_hi) {
 			const int rows = f.t_hi - f.t_lo + 1;
 			const long area = (long) (f.s_hi - f.s_lo + (DIRECT ? 0 : 1)) * (DIRECT ? rows | 1 : rows);
@@ -1355,7 +1413,7 @@ survey_kernel(const BackArgs a)
 	// wave reduce the count
 	for (int o = 32; o > 0; o >>= 1)
 		cnt += __shfl_xor(cnt, o, 64);
-	any = wave_max(any);
+	any = __any(any);
 	if (lane == 0) {
 		atomicAdd(a.count, cnt);
 		atomicMax(a.maxarea, maxarea);
@@ -1607,11 +1665,11 @@ static hipError_t launch_back_t(const BackArgs &a, size_t lds_bytes, hipStream_t
 	return hipGetLastError();
 }
 
-// two stage buffers of: slots + 8-word (view, column) records + the walk
+// two stage buffers of: slots + 6-word (view, column) records + the walk
 // modes' t_bin table + view headers (4-byte words)
 size_t back_lds_bytes(int nw, int vstage, int slot, int fmt)
 {
-	const size_t words = (size_t) vstage * slot + (size_t) vstage * 64 * 8
+	const size_t words = (size_t) vstage * slot + (size_t) vstage * 64 * 6
 		+ (fmt == FMT_F32 ? (size_t) vstage * nw * 64 : 0) + (size_t) vstage * 4;
 	return 2 * words * 4 + 2 * 4;   // two stage buffers and the zero words
 }

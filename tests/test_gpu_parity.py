@@ -321,6 +321,47 @@ def test_direct_all_configs_stored_views(device, waves, zper, fmt):
         assert err <= 1e-5, err
 
 
+@pytest.mark.parametrize("ds,ns", [(9.0, 12), (3.0, 40), (1.7, 75), (1.1, 120), (0.7, 180),
+                                   (0.4, 330), (0.35, 7)])
+def test_direct_staged_equals_gathered(device, ds, ns):
+    """FP16 footprints of 1 to about 50 detector columns per 8 x 8 tile (every
+    remainder of the staging batches, tiles across both detector edges, a
+    detector narrower than a footprint): views staged in LDS against the same
+    views gathered from HBM.  Both add the same terms; only the order of the 19
+    views changes where the small slot of the second plan still holds some of
+    them, hence 19 roundings of 2^-24."""
+    import torch
+    from mirt_amd import quantize_views
+    g = O.geom((41, 38, 22), (2.0, -2.0, 1.0), (0.25, 0.0, -0.5), 541.0, 949.0, 0.0,
+               ns, 37, (ds, 1.3), (0.25, 0.0))
+    proj = np.random.default_rng(ns).standard_normal((19, ns, 37)).astype(np.float32)
+    beta = np.linspace(0, 6, 19)
+    mask = np.ones((38, 41), np.uint8)
+    q, sc = quantize_views(torch.from_numpy(proj).to(device), "f16")
+    img = []
+    for cap in (0, 64):
+        plan = _plan(g, beta, mask, "f16")
+        plan.set_config(4, 16, 2, cap)
+        img.append(plan(q, sc).cpu().numpy())
+    assert np.any(img[1]) and O.rel_l2(img[0], img[1]) <= 19 * 2.0 ** -24
+
+
+def test_direct_wide_fan(device):
+    """An arc that reaches 61 degrees to each side (the arctangent's two forms
+    within a view), FP16 against FP64 of the stored views."""
+    import torch
+    from mirt_amd import quantize_views
+    g = O.geom((41, 38, 22), (11.0, -11.0, 1.0), (0.25, 0.0, -0.5), 420.0, 949.0, 0.0,
+               34, 37, (60.0, 1.3), (0.25, 0.0))
+    proj = np.random.default_rng(7).standard_normal((19, 34, 37)).astype(np.float32)
+    beta = np.linspace(0, 6, 19)
+    mask = np.ones((38, 41), np.uint8)
+    q, sc = quantize_views(torch.from_numpy(proj).to(device), "f16")
+    img = _plan(g, beta, mask, "f16")(q, sc).cpu().numpy()
+    want = O.back_ts_f64(g, _stored(q, sc), beta, mask)
+    assert np.any(want) and O.rel_l2(img, want) <= 1e-5
+
+
 @pytest.mark.parametrize("fmt", ["f16", "bf16"])
 def test_direct_hbm_gather_path(device, fmt):
     """Views whose footprint exceeds the LDS slot (a 128-word slot) gather from
