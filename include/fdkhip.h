@@ -238,9 +238,9 @@ int fdkhip_cbct_back_mat_direct(const fdkhip_geom *g, const void *proj_dev,
 /*
  * Device-resident 'fdk,ts,back': a plan holds the per-view tables, the
  * device mask and the launch configuration for one geometry and one view
- * list, so repeated backprojections of new projections cost one launch
- * sequence (replayed from a HIP graph after the first call).  No counterpart
- * object exists in the reference; the arithmetic is fdk_ts_back_t's.
+ * list, so repeated backprojections of new projections cost at most three
+ * launches.  No counterpart object exists in the reference; the arithmetic is
+ * fdk_ts_back_t's.
  *
  * fmt:  FDKHIP_F32 / F16 / BF16 storage of proj in fdkhip_plan_execute.
  * math: FDKHIP_MATH_EXACT or FDKHIP_MATH_FAST (F16/BF16 always use FAST).
@@ -274,7 +274,7 @@ int fdkhip_plan_create_helix(fdkhip_plan **plan, const fdkhip_geom *g, int32_t n
 int fdkhip_plan_execute(fdkhip_plan *plan, const void *proj_dev,
 	const float *scale_dev, float *image_dev, void *stream);
 
-/* Same as fdkhip_plan_execute but always launches directly (no graph). */
+/* Same as fdkhip_plan_execute. */
 int fdkhip_plan_execute_direct(fdkhip_plan *plan, const void *proj_dev,
 	const float *scale_dev, float *image_dev, void *stream);
 
@@ -341,8 +341,8 @@ int fdkhip_plan_profile(fdkhip_plan *plan, const void *proj_dev,
  * launch whose workgroups take (scan, column tile, z group) items from a
  * device work queue, so scans of uneven size keep every CU busy, or by one
  * launch per scan in turn (fdkhip_batch_set_per_scan), each in its own launch
- * shape; either way one graph replay per execute.  Each scan
- * i is what fdkhip_plan_execute would compute for geoms[i], na[i], beta[i]
+ * shape; either way one graph replay per execute where the buffers stay the
+ * same.  Each scan i is what fdkhip_plan_execute would compute for geoms[i], na[i], beta[i]
  * and mask[i] (mask may be NULL, or mask[i] NULL for all ones), with the same
  * result bits for the same math mode.  The reference backprojects one scan
  * per mex call (fbp/cbct_back.m:99-103) and has no batch object.
@@ -355,7 +355,8 @@ int fdkhip_batch_create(fdkhip_batch **batch, int32_t nscan,
 
 /* proj[i], scale[i] (F16/BF16 only; scale may be NULL for F32) and image[i]
  * are scan i's device buffers as in fdkhip_plan_execute.  Asynchronous on
- * `stream`; replayed from a HIP graph while the pointers stay the same. */
+ * `stream`; replayed from a HIP graph from the second call with the same
+ * pointers on. */
 int fdkhip_batch_execute(fdkhip_batch *batch, const void *const *proj,
 	const float *const *scale, float *const *image, void *stream);
 
