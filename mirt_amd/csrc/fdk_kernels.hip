@@ -88,7 +88,19 @@ enum { SETUP_OUT = 0, SETUP_ACTIVE = 1, SETUP_IDLE = 2 };
 struct ViewGeo {
 	float cosb, sinb, wzb;
 	int izb0, izb1;
+	bool axial;
 };
+
+// DIRECT (FP16/BF16) modes: the slice whose u each column's record holds.  On
+// an axial scan it is the slice next to the source's plane, where u is at
+// mid-detector for every column: u there and the products with slice
+// differences round least, and the same way whatever the z-group's height, so
+// that a launch's shape does not change its results.  On a helix, whose source
+// plane moves, the z-group's first slice.
+__device__ __forceinline__ int anchor_slice(const GeomF &g, bool axial, int zg0)
+{
+	return axial ? (int) fminf(fmaxf(rintf(g.wz), 0.f), (float) (g.nz - 1)) : zg0;
+}
 
 // Entry of a table that no kernel writes while it is read, at an index that is
 // the same in every lane: through the constant address space, so that it is a
@@ -105,7 +117,7 @@ typedef int vec2i __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ ViewGeo view_geo(const BackArgs &a, int v)
 {
 	const vec2f cs = table_entry(reinterpret_cast<const vec2f *>(a.trig), v);
-	ViewGeo vg{cs.x, cs.y, a.g.wz, 0, a.g.nz};
+	ViewGeo vg{cs.x, cs.y, a.g.wz, 0, a.g.nz, !a.vzs};
 	if (a.vzs) {
 		vg.wzb = a.g.wz + table_entry(a.vzs, v) / a.g.dz;
 		const vec2i w = table_entry(reinterpret_cast<const vec2i *>(a.izb), v);
@@ -305,9 +317,9 @@ __device__ __forceinline__ bool setup_walk(const GeomF &g, const ColSetup &c,
 // Slice range of one z-group for the FP16/BF16 paths, in u = t_bin + 1 (the
 // padded detector row coordinate, > 0 for every slice that reads a sample).
 // u is evaluated in closed form, as the consumer evaluates it:
-//   U0   = u(iz_min) + (zg0 - iz_min) * t_inc          (the group's first slice)
-//   U[k] = U0 + k * ZL * t_inc                          (chunk k's first slice)
-//   u    = U[k] + j * t_inc                             (slice zg0 + k*ZL + j)
+//   U0 = u(iz_min) + (za - iz_min) * t_inc       (the anchor slice za)
+//   U8 = U0 + (z8 - za) * t_inc                  (every eighth slice of the group)
+//   u  = U8 + j * t_inc                          (slice z8 + j)
 // each step one fmaf (one rounding each; nearer the exact value than the
 // reference's running sum).  [zlo, zhi) is [iz_min - 1, iz_max + 1) within
 // the group and the view's window: column_setup_fast's bounds are within one
@@ -322,11 +334,12 @@ __device__ __forceinline__ bool setup_direct(const GeomF &g, const ColSetup &c, 
 	int zg0, int zg1, float (&Uk)[NW], int &zlo, int &zhi, float &first, float &last)
 {
 	const float ti = c.t_inc;
-	const float U0 = fmaf((float) (zg0 - c.iz_min), ti, c.t_bin + 1.f);
+	const int za = anchor_slice(g, vg.axial, zg0);
+	const float U0 = fmaf((float) (za - c.iz_min), ti, c.t_bin + 1.f);
 	Uk[0] = U0;
 	auto uz = [&](int z) {           // z in [zg0, zg1)
-		const unsigned k = (unsigned) (z - zg0), j0 = k & ~(unsigned) (ZL - 1);
-		return fmaf((float) (k - j0), ti, fmaf((float) j0, ti, U0));
+		const int j = (z - zg0) & 7;
+		return fmaf((float) j, ti, fmaf((float) (z - j - za), ti, U0));
 	};
 	// the extra slice at each end stays inside the view's window (a helix)
 	const int lo = min(max(max(c.iz_min - 1, vg.izb0), zg0), zg1);
@@ -1019,8 +1032,15 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 	const float2 *Q2 = reinterpret_cast<const float2 *>(fdk_lds + bo + L.Q) + lane;
 	const int2 *VI = reinterpret_cast<const int2 *>(fdk_lds + bo + L.vinfo + 2);
 	const int *ZR = reinterpret_cast<const int *>(fdk_lds + bo + L.vinfo);
+	const int zrel = zg0 - anchor_slice(g, !WINDOW, zg0);
 	// relative to the z-group: chunk r starts at slice zoff(r)
 	auto zoff = [&](int r) { return (wave + r * NCW) * ZL; };
+	// U8: one fused multiply-add from the anchor for every eight slices, whatever
+	// the launch shape
+	const float zf = (float) (zrel + zoff(0));
+	auto u8 = [&](int r, int j, float ti, float U0) {
+		return fmaf(zf + (float) (r * NCW * ZL + (j & ~7)), ti, U0);
+	};
 	// window of chunk r relative to its first slice, clamped to [0, ZL]
 	auto window = [&](int2 wa, int r) {
 		const int zc = zg0 + zoff(r);
@@ -1058,7 +1078,10 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 			const int jhi = min(uhi - zoff(r), ZL);
 			if (jlo >= jhi)
 				continue;
-			const float t0 = fmaf((float) zoff(r), ti, p0.w);   // u at the chunk's first slice
+			float t8[ZL / 8];   // U8
+#pragma unroll
+			for (int k = 0; k < ZL / 8; ++k)
+				t8[k] = u8(r, 8 * k, ti, p0.w);
 			const int2 w = window(wa, r);
 			// halves of 4 slices; on helical plans groups of 8 (finer tests cost
 			// more than they save where windows cut groups)
@@ -1081,7 +1104,7 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 					float wu[HS];
 #pragma unroll
 					for (int k = 0; k < HS; ++k) {
-						const float u = __builtin_amdgcn_fmed3f(fmaf((float) (h0 + k), ti, t0),
+						const float u = __builtin_amdgcn_fmed3f(fmaf((float) ((h0 & 7) + k), ti, t8[h0 / 8]),
 							0.f, uh);
 						const int iu = (int) u;
 						wu[k] = __builtin_amdgcn_fractf(u);
@@ -1095,7 +1118,8 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 				} else {
 #pragma unroll
 					for (int j = h0; j < h0 + HS; ++j) {
-						const float u = __builtin_amdgcn_fmed3f(fmaf((float) j, ti, t0), 0.f, uh);
+						const float u = __builtin_amdgcn_fmed3f(fmaf((float) (j & 7), ti, t8[j / 8]),
+							0.f, uh);
 						acc[j] = slice_update_d<FMT>(acc[j], u, c1, wl, wr);
 					}
 				}
@@ -1132,15 +1156,16 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 				const int2 w = window(wa, r);
 				if (jlo >= jhi || (w.x <= 0 && w.y >= ZL))
 					continue;
-				const float t0 = fmaf((float) zoff(r), ti, p0.w);
 #pragma unroll
 				for (int g0 = 0; g0 < ZL; g0 += 8) {
 					if (g0 >= w.y || g0 + 8 <= w.x || (w.x <= g0 && g0 + 8 <= w.y)
 						|| g0 >= jhi || g0 + 8 <= jlo)
 						continue;
+					const float t8 = u8(r, g0, ti, p0.w);
 #pragma unroll
 					for (int j = g0; j < g0 + 8; ++j) {
-						const float u = __builtin_amdgcn_fmed3f(fmaf((float) j, ti, t0), 0.f, uh);
+						const float u = __builtin_amdgcn_fmed3f(fmaf((float) (j - g0), ti, t8),
+							0.f, uh);
 						const float up = slice_update_d<FMT>(acc[j], u, c1, wl, wr);
 						acc[j] = (j >= w.x && j < w.y) ? up : acc[j];
 					}
@@ -1172,11 +1197,11 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 			float (&acc)[ZL] = accs[r];
 			if (ulo >= zoff(r) + ZL || uhi <= zoff(r))
 				continue;
-			const float t0 = fmaf((float) zoff(r), ti, p0.w);
 			const int2 w = window(wa, r);
 #pragma unroll
 			for (int j = 0; j < ZL; ++j) {
-				const float u = __builtin_amdgcn_fmed3f(fmaf((float) j, ti, t0), 0.f, uh);
+				const float t8 = u8(r, j, ti, p0.w);
+				const float u = __builtin_amdgcn_fmed3f(fmaf((float) (j & 7), ti, t8), 0.f, uh);
 				const int iu = (int) u;
 				const float wu = __builtin_amdgcn_fractf(u);
 				const float up = bilerp_d(acc[j],
@@ -1289,10 +1314,12 @@ __device__ __forceinline__ void tile_pipeline(const BackArgs &a, int tile, int g
 // The second launch bound MW is the minimum waves per SIMD: 4 (at most 128
 // VGPRs), or 8 (at most 64) for a second build of the one-chunk FP16/BF16
 // kernels, whose small LDS stages can then let four 8-wave workgroups share
-// a CU; which one runs is a plan's choice (its autotuner times both).
+// a CU; which one runs is a plan's choice (its autotuner times both).  The
+// 48-slice FP16/BF16 kernels are held to 80 VGPRs, which lets three of their
+// workgroups share a CU (84 without the bound: clinical_arc FP16 9.4 ms for 7.7).
 // WIN: FP16/BF16 views of a helical plan (slice windows per view)
 template <int NW, int NP, int ZL, int FMT, bool FAST, int R, bool WIN, int MW>
-__global__ void __launch_bounds__((NW + NP) * 64, MW)
+__global__ void __launch_bounds__((NW + NP) * 64, (R == 3 && FMT != FMT_F32) ? 6 : MW)
 back_kernel(const BackArgs a)
 {
 	const int nblocks = a.ntiles * a.ngroups;

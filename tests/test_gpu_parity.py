@@ -230,6 +230,27 @@ def test_all_configs(device, waves, zper):
 
 
 @pytest.mark.parametrize("fmt", ["f16", "bf16"])
+@pytest.mark.parametrize("name", ["flat", "arc_tall", "wide_cone"])
+def test_16bit_bits_do_not_depend_on_shape(device, fmt, name):
+    """An axial FP16/BF16 plan evaluates the detector row of a slice from one
+    anchor slice whatever the z-group's height, so the default shape (chosen
+    from the geometry) and every other give the same bits while the
+    footprints fit the slots."""
+    import torch
+    from mirt_amd import quantize_views
+    g, proj, beta, mask = make_case(name, seed=31, data="noise")
+    q, sc = quantize_views(torch.from_numpy(proj).to(device), fmt)
+    plan = _plan(g, beta, mask, fmt)
+    assert plan.config["vstage"] > 0
+    want = plan(q, sc).cpu().numpy()
+    n = plan.count_updates()
+    for waves, zper in ((8, 16), (8, 8), (4, 8), (4, 16), (4, 48)):
+        plan.set_config(waves, zper, 2)
+        assert np.array_equal(plan(q, sc).cpu().numpy(), want), (waves, zper)
+        assert plan.count_updates() == n
+
+
+@pytest.mark.parametrize("fmt", ["f16", "bf16"])
 def test_occupancy_builds_same_bits(device, fmt):
     """The 8-waves-per-SIMD kernel build of one-chunk FP16/BF16 shapes gives
     the same bits as the 4-wave build (same instructions, other register
