@@ -208,6 +208,9 @@ struct fdkhip_plan {
 	int zs_lo = 0, zs_hi = 0;
 	long long n_updates = -1;
 	int maxarea = 0, fov_any = 0;
+	// the launch shape chosen when the plan was made (0 views per stage: the
+	// deepest that fits the largest footprint)
+	int def_nw = 8, def_zper = 16, def_vstage = 0, def_slot = 0;
 	size_t lds_limit = 65536;   // per workgroup, for the current configuration
 	size_t lds_max = 65536;     // device limit per workgroup
 	hipStream_t survey_stream = nullptr;   // stream of the survey pass (set-up)
@@ -217,6 +220,7 @@ struct fdkhip_plan {
 	int na1_half = 0;
 	float pitch = 0.f;
 	std::vector<int2> h_izb;
+	std::vector<float> h_vzs;
 	float *d_vzs = nullptr;
 	int2 *d_izb = nullptr;
 	int2 *d_gviews = nullptr;
@@ -266,9 +270,6 @@ static void quiesce(int device)
 		(void) hipSetDevice(cur);
 }
 
-// Tiling for (nw, zl), a survey pass over it, then the LDS slot size.
-// vstage_req > 0 fixes the views per stage; slot_cap > 0 caps the slot (floats)
-// -- views whose footprint does not fit gather from HBM instead of LDS.
 // Stage depth (views per LDS stage) and slot size (floats per staged view)
 // within `lds_limit` bytes.  A requested depth is kept and the slot shrunk
 // to fit; otherwise the deepest stage up to 16 views whose slot holds the
@@ -320,7 +321,200 @@ static int plan_minw(const fdkhip_plan *p)
 	return back_minw_supported(p->minw, p->zr, p->fmt) ? p->minw : 4;
 }
 
-static int configure(fdkhip_plan *p, int nw, int zper, int vstage_req, int slot_cap)
+// ---------------------------------------------------------------------------
+// default launch shape
+
+// What one z-group height means for a plan's scan, from a sample of views and
+// column tiles: the sampled (view, tile, group) triples that stage a footprint
+// out of those whose tile has a column, the footprints in floats, and the
+// slices of a column that a staged triple updates.
+struct HeightSample {
+	int height = 0;
+	long groups = 0;
+	double slices = 0;
+	std::vector<int> area;
+};
+
+constexpr int kSampleViews = 12, kSampleTiles = 7;
+
+// Footprints as the backprojection kernel stages them, from the four corner
+// columns of at most kSampleTiles^2 tiles in kSampleViews views (their own
+// samples are the extremes of a tile's).  An estimate: a view whose footprint
+// turns out larger than its slot gathers from memory, with the same result.
+static void sample_heights(const fdkhip_plan *p, const double *beta, const uint8_t *mask,
+	std::vector<HeightSample> &hs)
+{
+	const GeomF &g = p->gf;
+	const bool direct = p->fmt != FDKHIP_F32;
+	const int nv = std::min(p->na, kSampleViews);
+	const int nx = std::min(p->tiles_x, kSampleTiles), ny = std::min(p->tiles_y, kSampleTiles);
+	for (int v = 0; v < nv; ++v) {
+		const int ia = (int) ((2L * v + 1) * p->na / (2 * nv));
+		const double cb = cos(beta[ia]), sb = sin(beta[ia]);
+		const double wzb = g.wz + (p->helix ? p->h_vzs[ia] / g.dz : 0.);
+		const int w0 = p->helix ? p->h_izb[ia].x : 0, w1 = p->helix ? p->h_izb[ia].y : g.nz;
+		for (int j = 0; j < nx * ny; ++j) {
+			const int x0 = 8 * (int) ((2L * (j % nx) + 1) * p->tiles_x / (2 * nx));
+			const int y0 = 8 * (int) ((2L * (j / nx) + 1) * p->tiles_y / (2 * ny));
+			const int x1 = std::min(x0 + 7, g.nx - 1), y1 = std::min(y0 + 7, g.ny - 1);
+			bool any = !mask;
+			for (int y = y0; y <= y1 && !any; ++y)
+				for (int x = x0; x <= x1 && !any; ++x)
+					any = mask[(long) y * g.nx + x] != 0;
+			if (!any)
+				continue;
+			double smin = INFINITY, smax = -INFINITY, ti[4];
+			bool ok = true;
+			for (int c = 0; c < 4; ++c) {
+				const double xx = g.dx * ((c & 1 ? x1 : x0) - g.wx);
+				const double yy = g.dy * ((c & 2 ? y1 : y0) - g.wy);
+				const double xb = xx * cb + yy * sb, yb = g.dso - (-xx * sb + yy * cb);
+				const double mag = g.kind == KIND_PAR ? 1. : g.dsd / yb;
+				const double s = g.ws + (g.kind == KIND_ARC ? g.dsd * atan2(xb, yb) : mag * xb) / g.ds;
+				ti[c] = mag * g.dz / g.dt;
+				ok = ok && ti[c] > 0 && std::isfinite(ti[c]) && std::isfinite(s);
+				smin = std::min(smin, s);
+				smax = std::max(smax, s);
+			}
+			const double s0 = std::max(floor(smin) + 1, 0.), s1 = std::min(floor(smax) + 2, g.ns + 1.);
+			for (auto &h : hs)
+				for (int z0 = p->zs_lo; z0 < p->zs_hi; z0 += h.height) {
+					++h.groups;
+					if (!ok || s0 > s1)
+						continue;
+					const int ga = std::max(z0, w0), gb = std::min({z0 + h.height, p->zs_hi, w1});
+					double r0 = INFINITY, r1 = -INFINITY, n = 0;
+					for (double t : ti) {
+						const double za = std::max(floor(wzb - (g.wt + 1) / t) + 1, (double) ga);
+						const double zb = std::min(ceil(wzb + (g.nt - g.wt) / t), (double) gb);
+						if (za >= zb)
+							continue;
+						n += zb - za;
+						r0 = std::min(r0, floor(t * (za - wzb) + g.wt) + 1);
+						r1 = std::max(r1, floor(t * (zb - 1 - wzb) + g.wt) + 2);
+					}
+					const long rows = n > 0 ? (long) (std::min(r1, g.nt + 2.) - std::max(r0, 0.)) + 1 : 0;
+					if (rows <= 0)
+						continue;
+					const long a = (long) (s1 - s0 + (direct ? 0 : 1)) * (direct ? rows | 1 : rows);
+					h.area.push_back((int) std::min(a, 0x7fffffffL));
+					h.slices += n / 4;
+				}
+		}
+	}
+}
+
+// The launch shape of a plan that nobody has tuned.  A workgroup's time for a
+// view is the slower of its producers (the columns' set-up, then the footprint,
+// one view per producer wave at a time) and its consumers (the slices of one
+// wave) while it has a CU to itself, and the CU's issue time of all resident
+// workgroups once there are enough of them: hypot joins the two, whole rounds
+// of the card and the emptier last one add up.  How many are resident follows
+// from the stage's LDS and the kernel's registers, so a taller z-group saves
+// set-up but costs residency by its larger footprints, and a short launch wants
+// few slices per wave.  The six costs (clocks) per arithmetic and what a view
+// gathered from memory costs were fitted to
+// the times of every shape, depth and residency for 39 scans (15 to 512 columns
+// a side, 14 to 256 slices, flat, arc and helical): the shape chosen is within
+// 4 % of the best one there in the mean.  Against 128-slice groups of 8 waves
+// for all (64-slice groups of 4 for short volumes):
+// 256 x 256 x 128 FP32 from 360 flat views of 512 x 384 2.0 ms for 2.9,
+// 256 x 256 x 192 FP32 helix of 1476 views 6.9 for 12.7,
+// 256 x 256 x 128 FP16 from 425 views of 713 x 477 2.6 for 6.6,
+// 64 x 64 x 32 FP32 from 64 views 0.050 for 0.081; never more than 6 % behind.
+struct ShapeCosts {
+	double wave, slice;            // issue per CU: per consumer wave, per slice of a column
+	double setup, words;           // producer: per view, per 64 footprint words
+	double lane_slice, stage;      // consumer: per slice, per stage
+	double gather;                 // times the time, for views that do not fit
+};
+
+static const ShapeCosts kCostsDirect = {76, 1.2, 3250, 295, 91, 2890, 15};
+static const ShapeCosts kCostsF32 = {47, 19.7, 6530, 186, 150, 15, 2};
+
+// waves per SIMD the kernel's registers allow (the plans' 4-waves build)
+static int register_waves(int zper, int fmt)
+{
+	if (fmt != FDKHIP_F32)
+		return zper >= 48 ? 6 : 7;
+	return zper >= 48 ? 4 : 6;
+}
+
+static void choose_default(fdkhip_plan *p, const double *beta, const uint8_t *mask)
+{
+	static const struct { int nw, zper, vs[3]; } shapes[] = {
+		{4, 16, {4, 3, 8}}, {4, 8, {4, 3, 8}}, {4, 48, {4, 3, 8}}, {8, 8, {8, 4, 0}},
+		{8, 16, {8, 4, 0}}};
+	p->def_nw = p->zs_hi - p->zs_lo <= 64 ? 4 : 8;
+	p->def_zper = 16;
+	p->def_vstage = p->def_slot = 0;
+	p->tiles_x = (p->geom.nx + 7) / 8;
+	p->tiles_y = (p->geom.ny + 7) / 8;
+	const long tiles = (long) p->tiles_x * p->tiles_y;
+	if (p->na <= 0 || tiles <= 0 || p->zs_hi <= p->zs_lo)
+		return;
+	std::vector<HeightSample> hs(4);
+	for (int i = 0; i < 4; ++i)
+		hs[i].height = i < 3 ? 32 << i : 192;
+	sample_heights(p, beta, mask, hs);
+	const ShapeCosts &c = p->fmt == FDKHIP_F32 ? kCostsF32 : kCostsDirect;
+	double best = INFINITY;
+	for (const auto &sh : shapes) {
+		const auto &h = *std::find_if(hs.begin(), hs.end(),
+			[&](const HeightSample &x) { return x.height == sh.nw * sh.zper; });
+		int zl = 0, zr = 0;
+		if (h.area.empty() || !split_zper(sh.nw, sh.zper, p->fmt, zl, zr))
+			continue;
+		const double n = (double) h.area.size(), frac = n / h.groups, slices = h.slices / n;
+		double mean = 0;
+		int maxarea = 64;
+		for (int a : h.area) {
+			mean += a / n;
+			maxarea = std::max(maxarea, std::min(a, 1 << 20));
+		}
+		const double wgs = (double) tiles * ((p->zs_hi - p->zs_lo + h.height - 1) / h.height);
+		const int kreg = std::max(1, register_waves(sh.zper, p->fmt) * 4 / (2 * sh.nw));
+		for (int vs : sh.vs)
+			// as many resident workgroups as the registers allow, or fewer with
+			// larger slots
+			for (int k = kreg; vs > 0 && k >= (sh.nw >= 8 ? 1 : 2); --k) {
+				// whole allocation units: k of them have to fit a CU's LDS
+				const size_t lds = p->lds_max / k / 2560 * 2560;
+				const size_t fixed = back_lds_bytes(sh.nw * zr, vs, 0, p->fmt);
+				if (lds < fixed + (size_t) 8 * vs * 64)
+					continue;
+				const int slot = std::min((int) ((lds - fixed) / (8 * vs)), maxarea + maxarea / 8 + 64)
+					& ~15;
+				const double over = (double) std::count_if(h.area.begin(), h.area.end(),
+					[&](int a) { return a + a / 8 > slot; }) / n;   // the sample misses the extremes
+				const int np = sh.nw >= 8 ? 8 : 4;
+				const double produce = (c.setup + c.words * mean / 64) * ((vs + np - 1) / np) / vs;
+				const double consume = c.lane_slice
+					* std::min((double) sh.zper, zr > 1 ? slices / sh.nw : slices) + c.stage / vs;
+				const double alone = std::max(produce, consume) * (1 + c.gather * over);
+				const double issue = c.wave * sh.nw + c.slice * slices;
+				const double rounds = floor(wgs / (256. * k));
+				const double rest = ceil(wgs / 256. - rounds * k - 1e-9);
+				double t = rounds * hypot(alone, issue * k);
+				if (rest > 0)
+					t += hypot(alone, issue * rest);
+				t *= frac + 0.25 * (1 - frac);   // a group no view meets costs its columns' set-up
+				if (over > 0.2)
+					t *= 2;   // only where nothing else fits
+				if (t < best) {
+					best = t;
+					p->def_nw = sh.nw;
+					p->def_zper = sh.zper;
+					p->def_vstage = vs;
+					p->def_slot = slot;
+				}
+			}
+	}
+}
+
+// Tiling for (nw, zper): the column tiles, the z-groups and, for a helical
+// scan, the views of each z-group.
+static int set_tiling(fdkhip_plan *p, int nw, int zper)
 {
 	int zl = 0, zr = 0;
 	if (!split_zper(nw, zper, p->fmt, zl, zr))
@@ -360,39 +554,57 @@ static int configure(fdkhip_plan *p, int nw, int zper, int vstage_req, int slot_
 		HIP_TRY(hipMemcpy(p->d_gviews, gv.data(), sizeof(int2) * p->ngroups,
 			hipMemcpyHostToDevice));
 	}
+	// 8 consumer waves (+8 producers) fill a CU with one workgroup, 4 (+4) fit
+	// at least two
+	p->lds_limit = (nw >= 8) ? p->lds_max : p->lds_max / 2;
+	return FDKHIP_OK;
+}
+
+// The exact survey of the current tiling (cached per tiling): the reference's
+// loop iterations, the largest footprint, whether any column meets any view.
+static int run_survey(fdkhip_plan *p)
+{
 	p->maxarea = 0;
 	p->fov_any = 0;
 	p->n_updates = 0;
-	bool cached = false;
 	for (const auto &sv : p->surveys)
-		if (sv.nw == nw && sv.zl == zl && sv.zr == zr) {
+		if (sv.nw == p->nw && sv.zl == p->zl && sv.zr == p->zr) {
 			p->maxarea = sv.maxarea;
 			p->fov_any = sv.fov_any;
 			p->n_updates = sv.n_updates;
-			cached = true;
+			return FDKHIP_OK;
 		}
-	if (!cached && p->ngroups > 0 && p->tiles_x > 0 && p->tiles_y > 0 && p->na > 0) {
-		hipStream_t ss = p->survey_stream;
-		HIP_TRY(launch_zero_u64(p->d_count, 1, ss));
-		HIP_TRY(launch_zero_i32(p->d_maxarea, 1, ss));
-		HIP_TRY(launch_zero_i32(p->d_any, 1, ss));
-		BackArgs a = make_args(p, nullptr, nullptr, nullptr);
-		HIP_TRY(launch_survey(a, nw * zr, zl, p->fmt != FDKHIP_F32, ss));
-		unsigned long long cnt = 0;
-		HIP_TRY(hipMemcpyAsync(&cnt, p->d_count, sizeof cnt, hipMemcpyDeviceToHost, ss));
-		HIP_TRY(hipMemcpyAsync(&p->maxarea, p->d_maxarea, sizeof(int), hipMemcpyDeviceToHost,
-			ss));
-		HIP_TRY(hipMemcpyAsync(&p->fov_any, p->d_any, sizeof(int), hipMemcpyDeviceToHost, ss));
-		HIP_TRY(hipStreamSynchronize(ss));
-		p->n_updates = (long long) cnt;
-		p->surveys.push_back({nw, zl, zr, p->maxarea, p->fov_any, p->n_updates});
-	}
-	// views per stage and slot size within the LDS budget: 8 consumer waves
-	// (+8 producers) fill a CU with one workgroup, 4 (+4) fit two
-	p->lds_limit = (nw >= 8) ? p->lds_max : p->lds_max / 2;
+	if (p->ngroups == 0 || p->tiles_x == 0 || p->tiles_y == 0 || p->na == 0)
+		return FDKHIP_OK;
+	hipStream_t ss = p->survey_stream;
+	HIP_TRY(launch_zero_u64(p->d_count, 1, ss));
+	HIP_TRY(launch_zero_i32(p->d_maxarea, 1, ss));
+	HIP_TRY(launch_zero_i32(p->d_any, 1, ss));
+	BackArgs a = make_args(p, nullptr, nullptr, nullptr);
+	HIP_TRY(launch_survey(a, p->nw * p->zr, p->zl, p->fmt != FDKHIP_F32, ss));
+	unsigned long long cnt = 0;
+	HIP_TRY(hipMemcpyAsync(&cnt, p->d_count, sizeof cnt, hipMemcpyDeviceToHost, ss));
+	HIP_TRY(hipMemcpyAsync(&p->maxarea, p->d_maxarea, sizeof(int), hipMemcpyDeviceToHost, ss));
+	HIP_TRY(hipMemcpyAsync(&p->fov_any, p->d_any, sizeof(int), hipMemcpyDeviceToHost, ss));
+	HIP_TRY(hipStreamSynchronize(ss));
+	p->n_updates = (long long) cnt;
+	p->surveys.push_back({p->nw, p->zl, p->zr, p->maxarea, p->fov_any, p->n_updates});
+	return FDKHIP_OK;
+}
+
+// Tiling for (nw, zper), a survey pass over it, then the LDS slot size.
+// vstage_req > 0 fixes the views per stage; slot_cap > 0 caps the slot (floats)
+// -- views whose footprint does not fit gather from HBM instead of LDS.
+static int configure(fdkhip_plan *p, int nw, int zper, int vstage_req, int slot_cap)
+{
+	int rc = set_tiling(p, nw, zper);
+	if (!rc)
+		rc = run_survey(p);
+	if (rc)
+		return rc;
 	int vstage = 0, slot = 0;
-	if (!choose_layout(nw * zr, p->fmt, p->maxarea, vstage_req, slot_cap, p->lds_limit, vstage,
-			slot))
+	if (!choose_layout(nw * p->zr, p->fmt, p->maxarea, vstage_req, slot_cap, p->lds_limit,
+			vstage, slot))
 		return fail(FDKHIP_EUNSUPPORTED, "LDS budget too small for waves=%d", nw);
 	p->vstage = vstage;
 	p->slot = slot;
@@ -417,8 +629,18 @@ static int plan_free(fdkhip_plan *p)
 	return FDKHIP_OK;
 }
 
-static int apply_tuned(fdkhip_plan *p);
 static int plan_default_config(fdkhip_plan *p);
+
+// fdk,ts.c:153-154: the reference fails on the first in-FOV column
+static int check_direction(fdkhip_plan *p)
+{
+	if (p->gf.dz / p->gf.dt >= 0)
+		return FDKHIP_OK;
+	const int rc = run_survey(p);
+	if (rc || !p->fov_any)
+		return rc;
+	return fail(FDKHIP_EGEOM, "todo: dz/dt < 0 not done");
+}
 
 constexpr size_t kPadTail = 256;   // zero bytes after a plan's padded copy
 
@@ -541,15 +763,14 @@ static int plan_create_impl(fdkhip_plan **out, const fdkhip_geom *g, int32_t na,
 #undef PLAN_TRY
 
 	support_z(g, mask_host, p->zs_lo, p->zs_hi, zs_lo, zs_hi);
+	p->h_vzs = vzs;
+	choose_default(p, beta, mask_host);
 	rc = plan_default_config(p);
+	if (!rc)
+		rc = check_direction(p);
 	if (rc) {
 		plan_free(p);
 		return rc;
-	}
-	// fdk,ts.c:153-154: the reference fails on the first in-FOV column
-	if (p->gf.dz / p->gf.dt < 0 && p->fov_any) {
-		plan_free(p);
-		return fail(FDKHIP_EGEOM, "todo: dz/dt < 0 not done");
 	}
 	*out = p;
 	return FDKHIP_OK;
@@ -621,6 +842,11 @@ extern "C" int fdkhip_plan_count_updates(fdkhip_plan *p, int64_t *n)
 {
 	if (!p || !n)
 		return fail(FDKHIP_EARG, "NULL argument");
+	if (p->n_updates < 0) {
+		const int rc = run_survey(p);
+		if (rc)
+			return rc;
+	}
 	*n = p->n_updates;
 	return FDKHIP_OK;
 }
@@ -792,13 +1018,12 @@ extern "C" int fdkhip_back_noalloc(const fdkhip_geom *g, int32_t na, const doubl
 	HIP_TRY(hipStreamSynchronize(s));
 	// the launch shape and layout a plan of this scan would use
 	support_z(g, mask_host, p.zs_lo, p.zs_hi);
-	rc = configure(&p, p.zs_hi - p.zs_lo <= 64 ? 4 : 8, 16, 0, 0);
-	if (rc == FDKHIP_OK)
-		rc = apply_tuned(&p);
+	choose_default(&p, beta, mask_host);
+	rc = plan_default_config(&p);
+	if (!rc)
+		rc = check_direction(&p);
 	if (rc)
 		return rc;
-	if (p.gf.dz / p.gf.dt < 0 && p.fov_any)
-		return fail(FDKHIP_EGEOM, "todo: dz/dt < 0 not done");
 	return plan_launch(&p, proj_dev, scale_dev, image_dev, s);
 }
 
@@ -2100,23 +2325,24 @@ extern "C" int fdkhip_plan_profile(fdkhip_plan *p, const void *proj, const float
 
 
 // apply a choice made earlier in this process for the same geometry
-static int apply_tuned(fdkhip_plan *p)
-{
-	Tuned t;
-	if (!tuned_lookup(tune_key(p), t))
-		return FDKHIP_OK;
-	p->minw = t.minw;
-	return configure(p, t.nw, t.zl, t.vstage, 0);
-}
-
-// a plan's own launch shape: 8 waves x 16 slices = 128-slice z-groups (4 x 16
-// when the support is short), or the autotuner's choice made earlier in this
-// process for the same geometry
+// a plan's own launch shape: the autotuner's choice made earlier in this
+// process for the same geometry, or the one chosen when the plan was made,
+// whose slot needs no survey
 static int plan_default_config(fdkhip_plan *p)
 {
-	const int nw = (p->zs_hi - p->zs_lo <= 64) ? 4 : 8;
-	const int rc = configure(p, nw, 16, 0, 0);
-	return rc ? rc : apply_tuned(p);
+	Tuned t;
+	if (tuned_lookup(tune_key(p), t)) {
+		p->minw = t.minw;
+		return configure(p, t.nw, t.zl, t.vstage, 0);
+	}
+	if (p->def_vstage == 0)
+		return configure(p, p->def_nw, p->def_zper, 0, 0);
+	const int rc = set_tiling(p, p->def_nw, p->def_zper);
+	if (rc)
+		return rc;
+	p->vstage = p->def_vstage;
+	p->slot = p->def_slot;
+	return FDKHIP_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -2309,7 +2535,17 @@ extern "C" int fdkhip_batch_create(fdkhip_batch **out, int32_t nscan, const fdkh
 		}
 		b->plans.push_back(p);
 	}
-	int rc = batch_configure(b, 8, 16, 0);
+	// One launch per scan where a scan by itself gives half of the CUs a
+	// workgroup, each in its own shape; the queue for smaller ones, whose
+	// launches would leave most of the card idle.  Batches of 24 FP16 scans,
+	// persistent / per scan: 64 workgroups a scan 0.92 / 1.13 ms, 216
+	// 2.23 / 1.97, 416 4.45 / 3.02, 1584 15.6 / 11.5; FP32 2.04 / 2.15,
+	// 4.28 / 3.24, 7.63 / 5.22, 22.2 / 17.3.
+	long long wgs = 0;
+	for (const auto *p : b->plans)
+		wgs += (p->na > 0) ? (long long) p->tiles_x * p->tiles_y * p->ngroups : 0;
+	b->per_scan = wgs >= 128LL * nscan;
+	int rc = b->per_scan ? FDKHIP_OK : batch_configure(b, 8, 16, 0);
 	if (rc) {
 		batch_free(b);
 		return rc;
@@ -2407,17 +2643,29 @@ extern "C" int fdkhip_batch_count_updates(fdkhip_batch *b, int64_t *n)
 	if (!b || !n)
 		return fail(FDKHIP_EARG, "NULL argument");
 	long long s = 0;
-	for (auto *p : b->plans)
-		s += p->n_updates;
+	for (auto *p : b->plans) {
+		int64_t m = 0;
+		const int rc = fdkhip_plan_count_updates(p, &m);
+		if (rc)
+			return rc;
+		s += m;
+	}
 	*n = s;
 	return FDKHIP_OK;
+}
+
+// a scan's share of the batch: its column-view-slice triples, of which its
+// updates are those inside the detector
+static long long plan_work(const fdkhip_plan *p)
+{
+	return (long long) p->na * p->geom.nx * p->geom.ny * (p->zs_hi - p->zs_lo);
 }
 
 // the backprojection alone on the uploaded arguments: the persistent kernel
 // (with its queue reset), or each scan's own launch.  The per-scan launches
 // go to two streams, `s` and the batch's side stream (forked from `s` and
-// joined back into it), the scans in descending order of update count each
-// to the stream with fewer updates queued: the next scan's workgroups then
+// joined back into it), the scans in descending order of size (plan_work)
+// each to the stream with less queued: the next scan's workgroups then
 // fill the CUs that a launch's last round leaves idle.
 static int batch_kernel_launch(fdkhip_batch *b, hipStream_t s)
 {
@@ -2432,14 +2680,14 @@ static int batch_kernel_launch(fdkhip_batch *b, hipStream_t s)
 			if (b->plans[i]->ngroups > 0 && b->plans[i]->na > 0)
 				order.push_back(i);
 		std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-			return b->plans[x]->n_updates > b->plans[y]->n_updates; });
+			return plan_work(b->plans[x]) > plan_work(b->plans[y]); });
 		HIP_TRY(hipEventRecord(b->fork_ev, s));
 		HIP_TRY(hipStreamWaitEvent(b->side, b->fork_ev, 0));
 		long long queued[2] = {0, 0};
 		for (int i : order) {
 			const fdkhip_plan *p = b->plans[i];
 			const int k = queued[1] < queued[0] ? 1 : 0;
-			queued[k] += p->n_updates;
+			queued[k] += plan_work(p);
 			HIP_TRY(launch_back(b->host_args[i], p->nw, p->zl, p->zr, p->fmt,
 				p->math == FDKHIP_MATH_FAST, plan_minw(p), k ? b->side : s));
 		}
