@@ -1467,21 +1467,37 @@ __global__ void fill_kernel(float *image, long ncol, int nz, int zlo, int zhi)
 }
 
 // zero-padded copy of the views: [na][ns][nt] -> [na][ns+2][nt+2] (the
-// one-sample zero border of fdk_ts_put_view, fdk,ts,t.c:13-21, for all views)
-template <typename T>
-__global__ void pad_kernel(const T *src, T *dst, int ns, int nt, long total)
+// one-sample zero border of fdk_ts_put_view, fdk,ts,t.c:13-21, for all views).
+// Bound by memory.  A wave copies 512 consecutive words of the padded array:
+// the place of the first is one scalar division, the other lanes and words
+// step from it (two 64-bit divisions per word: 360 views of 512 x 384 0.164 ms
+// for 0.137, 1476 of 888 x 64 0.192 for 0.162).  A wave per column is slower
+// where columns are short (0.142 and 0.259).
+constexpr int PAD_WORDS = 512;
+__global__ void __launch_bounds__(256)
+pad_kernel(const float *src, float *dst, int ns, int nt, long total)
 {
-	const int pnt = nt + 2, pns = ns + 2;
-	for (long i = (long) blockIdx.x * blockDim.x + threadIdx.x; i < total;
-		i += (long) gridDim.x * blockDim.x) {
-		const int t = (int) (i % pnt);
-		const long q = i / pnt;
-		const int s = (int) (q % pns);
-		const long v = q / pns;
-		T val = T(0);
-		if (s >= 1 && s <= ns && t >= 1 && t <= nt)
-			val = src[(v * ns + (s - 1)) * nt + (t - 1)];
-		dst[i] = val;
+	const int pnt = nt + 2, pns = ns + 2, lane = threadIdx.x & 63;
+	const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
+	const long step = (long) gridDim.x * 4 * PAD_WORDS;
+	for (long b = ((long) blockIdx.x * 4 + wave) * PAD_WORDS; b < total; b += step) {
+		const long q = b / pnt;
+		long v = q / pns;
+		int t = (int) (b - q * pnt) + lane, s = (int) (q - v * pns);
+#pragma unroll
+		for (int j = 0; j < PAD_WORDS; j += 64, t += 64) {
+			while (t >= pnt) {
+				t -= pnt;
+				if (++s == pns) {
+					s = 0;
+					++v;
+				}
+			}
+			if (b + j + lane >= total)
+				break;
+			const bool in = s >= 1 && s <= ns && t >= 1 && t <= nt;
+			dst[b + j + lane] = in ? src[(v * ns + (s - 1)) * nt + (t - 1)] : 0.f;
+		}
 	}
 }
 
@@ -1862,8 +1878,8 @@ hipError_t launch_fill(float *image, long ncol, int nz, int zlo, int zhi, hipStr
 hipError_t launch_pad(const float *src, float *dst, int ns, int nt, int na, hipStream_t s)
 {
 	const long total = (long) na * (ns + 2) * (nt + 2);
-	const int blocks = (int) min((total + 255) / 256, (long) 8192);
-	hipLaunchKernelGGL(pad_kernel<float>, dim3(blocks), dim3(256), 0, s, src, dst, ns, nt, total);
+	const int blocks = (int) min((total + 4 * PAD_WORDS - 1) / (4 * PAD_WORDS), (long) 65536);
+	hipLaunchKernelGGL(pad_kernel, dim3(blocks), dim3(256), 0, s, src, dst, ns, nt, total);
 	return hipGetLastError();
 }
 
