@@ -553,7 +553,8 @@ class FdkPlan:
 
 
 class FdkBatch:
-    """Many scans backprojected by one persistent launch (libfdkhip batch).
+    """Many scans backprojected in one execute (libfdkhip batch): one launch per
+    scan where the scans are large, else one persistent launch.
 
     ``scans`` is a sequence of ``(geom, beta, mask)`` (mask may be None).
     :meth:`__call__` takes per-scan device projections (and scales for
