@@ -91,15 +91,19 @@ struct ViewGeo {
 	bool axial;
 };
 
-// DIRECT (FP16/BF16) modes: the slice whose u each column's record holds.  On
-// an axial scan it is the slice next to the source's plane, where u is at
-// mid-detector for every column: u there and the products with slice
-// differences round least, and the same way whatever the z-group's height, so
-// that a launch's shape does not change its results.  On a helix, whose source
-// plane moves, the z-group's first slice.
-__device__ __forceinline__ int anchor_slice(const GeomF &g, bool axial, int zg0)
+// DIRECT (FP16/BF16) modes: the z coordinate at which each column's record holds
+// u.  On an axial scan it is the half slice nearest to the source's plane: u is
+// wt + 1 in that plane, so it takes no rounding of the column's own where the
+// plane is at a half slice and one elsewhere; distances from it are exact, and a
+// slice's u has the roundings of its own two fused multiply-adds, the same
+// whatever the z-group's height: a launch's shape does not change its results.
+// (512 rows, 128 slices that reach at most both ends of the detector, emulated in
+// FP32: rms error of u 0.95e-5 rows; 1.2e-5 from the z-group's first slice, 1.4e-5
+// from the slice next to the source's plane with u carried there from the cone's
+// lower edge.)  On a helix, whose source plane moves, the z-group's first slice.
+__device__ __forceinline__ float anchor_z(const GeomF &g, bool axial, int zg0)
 {
-	return axial ? (int) fminf(fmaxf(rintf(g.wz), 0.f), (float) (g.nz - 1)) : zg0;
+	return axial ? 0.5f * rintf(2.f * g.wz) : (float) zg0;
 }
 
 // Entry of a table that no kernel writes while it is read, at an index that is
@@ -114,11 +118,11 @@ __device__ __forceinline__ T table_entry(const T *p, int i)
 typedef float vec2f __attribute__((ext_vector_type(2)));
 typedef int vec2i __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ ViewGeo view_geo(const BackArgs &a, int v)
+__device__ __forceinline__ ViewGeo view_geo(const BackArgs &a, int v, bool helix)
 {
 	const vec2f cs = table_entry(reinterpret_cast<const vec2f *>(a.trig), v);
-	ViewGeo vg{cs.x, cs.y, a.g.wz, 0, a.g.nz, !a.vzs};
-	if (a.vzs) {
+	ViewGeo vg{cs.x, cs.y, a.g.wz, 0, a.g.nz, !helix};
+	if (helix) {
 		vg.wzb = a.g.wz + table_entry(a.vzs, v) / a.g.dz;
 		const vec2i w = table_entry(reinterpret_cast<const vec2i *>(a.izb), v);
 		vg.izb0 = w.x;
@@ -317,8 +321,9 @@ __device__ __forceinline__ bool setup_walk(const GeomF &g, const ColSetup &c,
 // Slice range of one z-group for the FP16/BF16 paths, in u = t_bin + 1 (the
 // padded detector row coordinate, > 0 for every slice that reads a sample).
 // u is evaluated in closed form, as the consumer evaluates it:
-//   U0 = u(iz_min) + (za - iz_min) * t_inc       (the anchor slice za)
-//   U8 = U0 + (z8 - za) * t_inc                  (every eighth slice of the group)
+//   U0 = wt + 1 + (anchor_z - wz) * t_inc, or on a helix
+//        u(iz_min) + (zg0 - iz_min) * t_inc
+//   U8 = U0 + (z8 - anchor_z) * t_inc            (every eighth slice of the group)
 //   u  = U8 + j * t_inc                          (slice z8 + j)
 // each step one fmaf (one rounding each; nearer the exact value than the
 // reference's running sum).  [zlo, zhi) is [iz_min - 1, iz_max + 1) within
@@ -334,12 +339,13 @@ __device__ __forceinline__ bool setup_direct(const GeomF &g, const ColSetup &c, 
 	int zg0, int zg1, float (&Uk)[NW], int &zlo, int &zhi, float &first, float &last)
 {
 	const float ti = c.t_inc;
-	const int za = anchor_slice(g, vg.axial, zg0);
-	const float U0 = fmaf((float) (za - c.iz_min), ti, c.t_bin + 1.f);
+	const float za = anchor_z(g, vg.axial, zg0);
+	const float U0 = vg.axial ? fmaf(za - g.wz, ti, g.wt + 1.f)
+		: fmaf((float) (zg0 - c.iz_min), ti, c.t_bin + 1.f);
 	Uk[0] = U0;
 	auto uz = [&](int z) {           // z in [zg0, zg1)
 		const int j = (z - zg0) & 7;
-		return fmaf((float) j, ti, fmaf((float) (z - j - za), ti, U0));
+		return fmaf((float) j, ti, fmaf((float) (z - j) - za, ti, U0));
 	};
 	// the extra slice at each end stays inside the view's window (a helix)
 	const int lo = min(max(max(c.iz_min - 1, vg.izb0), zg0), zg1);
@@ -600,7 +606,7 @@ __device__ __forceinline__ void stage_pairs(const uint16_t *view, const GeomF &g
 // before the stage barrier; DIRECT (FP16/BF16) stages column pairs from the
 // caller's views (stage_pairs).  R: chunks per consumer wave (the walk
 // modes' consumers test slice groups against the tile's ranges with R > 1).
-template <int NW, int NP, int ZL, int FMT, bool FAST, int R>
+template <int NW, int NP, int ZL, int FMT, bool FAST, int R, bool WIN>
 __device__ __forceinline__ void produce(const BackArgs &a, int bo,
 	const Lds<NW, FMT == FMT_F32> &L,
 	int v0, int nv, int pw, int lane, bool colvalid, float xx, float yy, int zg0, int zg1)
@@ -613,7 +619,7 @@ __device__ __forceinline__ void produce(const BackArgs &a, int bo,
 		// col_range, and its record must still describe an empty range
 		ColRange cr{};
 		float Tk[NW] = {};
-		const ViewGeo vg = view_geo(a, v);
+		const ViewGeo vg = view_geo(a, v, DIRECT ? WIN : a.vzs != nullptr);
 		const bool act = colvalid
 			&& col_range<NW, ZL, DIRECT>(g, xx, yy, vg, zg0, zg1, cr, Tk);
 		const ColSetup &c = cr.c;
@@ -1032,12 +1038,12 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 	const float2 *Q2 = reinterpret_cast<const float2 *>(fdk_lds + bo + L.Q) + lane;
 	const int2 *VI = reinterpret_cast<const int2 *>(fdk_lds + bo + L.vinfo + 2);
 	const int *ZR = reinterpret_cast<const int *>(fdk_lds + bo + L.vinfo);
-	const int zrel = zg0 - anchor_slice(g, !WINDOW, zg0);
+	const float za = anchor_z(g, !WINDOW, zg0);
 	// relative to the z-group: chunk r starts at slice zoff(r)
 	auto zoff = [&](int r) { return (wave + r * NCW) * ZL; };
 	// U8: one fused multiply-add from the anchor for every eight slices, whatever
 	// the launch shape
-	const float zf = (float) (zrel + zoff(0));
+	const float zf = (float) (zg0 + zoff(0)) - za;
 	auto u8 = [&](int r, int j, float ti, float U0) {
 		return fmaf(zf + (float) (r * NCW * ZL + (j & ~7)), ti, U0);
 	};
@@ -1258,14 +1264,14 @@ __device__ __forceinline__ void tile_pipeline(const BackArgs &a, int tile, int g
 		if (FMT != FMT_F32 && pw == 0 && lane < 2)
 			fdk_lds[L.zero + lane] = 0.f;   // read by DIRECT lanes without work
 		if (nstage > 0)
-			produce<NC, NP, ZL, FMT, FAST, R>(a, 0, L, va, min(a.vstage, vb - va), pw, lane,
+			produce<NC, NP, ZL, FMT, FAST, R, WIN>(a, 0, L, va, min(a.vstage, vb - va), pw, lane,
 				colvalid, xx, yy, zg0, zg1);
 		__builtin_amdgcn_s_waitcnt(0);   // staged footprints have landed in LDS
 		__syncthreads();
 		for (int s = 0; s < nstage; ++s) {
 			if (s + 1 < nstage) {
 				const int v0 = va + (s + 1) * a.vstage;
-				produce<NC, NP, ZL, FMT, FAST, R>(a, ((s + 1) & 1) * L.total, L, v0,
+				produce<NC, NP, ZL, FMT, FAST, R, WIN>(a, ((s + 1) & 1) * L.total, L, v0,
 					min(a.vstage, vb - v0), pw, lane, colvalid, xx, yy, zg0, zg1);
 			}
 			__builtin_amdgcn_s_waitcnt(0);
@@ -1418,7 +1424,7 @@ survey_kernel(const BackArgs a)
 	unsigned long long cnt = 0;
 	int maxarea = 0, any = 0;
 	for (int v = 0; v < g.na; ++v) {
-		const ViewGeo vg = view_geo(a, v);
+		const ViewGeo vg = view_geo(a, v, a.vzs != nullptr);
 		ColSetup c;
 		const int code = colvalid ? column_setup(g, xx, yy, vg, c) : SETUP_OUT;
 		any |= (code != SETUP_OUT) ? 1 : 0;

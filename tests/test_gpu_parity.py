@@ -251,6 +251,35 @@ def test_16bit_bits_do_not_depend_on_shape(device, fmt, name):
 
 
 @pytest.mark.parametrize("fmt", ["f16", "bf16"])
+@pytest.mark.parametrize("dz", [0.7, 1.1, 1.3, 1.9])
+def test_16bit_row_coordinate_rounding(device, dz, fmt):
+    """A slice's detector row on a tall detector: one parallel view of rows of
+    alternating sign (the image is then 1 - 2 fract(u) up to its sign), no
+    rounding of the step or along s.  The row is two fused multiply-adds from
+    the source's plane -- to the slice's group of eight, to the slice -- so it
+    is off by half a unit in the last place of each at most, and the image by
+    twice that and its own rounding (2^-24)."""
+    import torch
+    nt, nz = 512, 256
+    g = O.geom((8, 8, nz), (1.0, -1.0, dz), (0, 0, 0), np.inf, np.inf, 0.0,
+               16, nt, (1.0, 1.0), (0.0, 0.0))
+    dtype = {"f16": torch.float16, "bf16": torch.bfloat16}[fmt]
+    sign = (1.0 - 2.0 * (np.arange(nt) % 2)).astype(np.float32)
+    q = torch.from_numpy(np.broadcast_to(sign, (1, 16, nt)).copy()).to(device, dtype)
+    img = _plan(g, np.zeros(1), np.ones((8, 8), np.uint8), fmt)(
+        q, torch.ones(1, device=device)).cpu().numpy()
+    z = np.arange(nz)
+    row = lambda zz: nt / 2 + 0.5 + (zz - (nz - 1) / 2) * float(np.float32(dz))   # noqa: E731
+    u, u8 = row(z), row(z & ~7)
+    assert u.min() > 1 and u.max() < nt
+    want = np.where(np.floor(u) % 2 == 1, 1.0, -1.0) * (1 - 2 * (u - np.floor(u)))
+    half = lambda x: np.spacing(x.astype(np.float32)).astype(np.float64) / 2      # noqa: E731
+    tol = 2 * (half(u8) + half(u)) + 2.0 ** -24
+    err = np.abs(img - want)
+    assert np.all(err <= tol), (err / tol).max()
+
+
+@pytest.mark.parametrize("fmt", ["f16", "bf16"])
 def test_occupancy_builds_same_bits(device, fmt):
     """The 8-waves-per-SIMD kernel build of one-chunk FP16/BF16 shapes gives
     the same bits as the 4-wave build (same instructions, other register
