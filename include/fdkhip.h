@@ -287,6 +287,8 @@ int fdkhip_plan_config(const fdkhip_plan *plan, int32_t cfg[6]);
  * must be a pair the build supports; vstage (views per LDS stage) and
  * slot_cap (largest staged footprint, floats) are upper bounds, 0 = chosen
  * automatically.  Views whose footprint exceeds the slot gather from HBM.
+ * Results do not depend on the configuration, except that an FP16/BF16 helical
+ * plan may add a slice's views in another order (FP32 rounding).
  * fdkhip_plan_config shows what was taken. */
 int fdkhip_plan_set_config(fdkhip_plan *plan, int32_t waves, int32_t zper,
 	int32_t vstage, int32_t slot_cap);
@@ -380,8 +382,8 @@ int fdkhip_batch_config(const fdkhip_batch *batch, int32_t cfg[6]);
  * with its neighbouring tiles, which then share their detector footprints
  * in L2; the persistent kernel's workgroups drift apart from item to item.
  * fdkhip_batch_set_config and fdkhip_batch_set_zper return to the
- * persistent kernel.  Results: the same bits as the persistent kernel for
- * EXACT.  No reference counterpart (a launch parameter of the batch). */
+ * persistent kernel.  Results: the same bits as the persistent kernel.  No
+ * reference counterpart (a launch parameter of the batch). */
 int fdkhip_batch_set_per_scan(fdkhip_batch *batch);
 
 /* Launch shape for the whole batch (a pair the build supports) and an upper

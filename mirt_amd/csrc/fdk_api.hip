@@ -340,7 +340,8 @@ constexpr int kSampleViews = 12, kSampleTiles = 7;
 // Footprints as the backprojection kernel stages them, from the four corner
 // columns of at most kSampleTiles^2 tiles in kSampleViews views (their own
 // samples are the extremes of a tile's).  An estimate: a view whose footprint
-// turns out larger than its slot gathers from memory, with the same result.
+// turns out larger than its slot gathers from memory, added in its turn with the
+// same bits (an FP16/BF16 helix: with sums in another order, see consume_direct).
 static void sample_heights(const fdkhip_plan *p, const double *beta, const uint8_t *mask,
 	std::vector<HeightSample> &hs)
 {

@@ -1009,11 +1009,14 @@ __device__ __forceinline__ int2 view_window(const BackArgs &a, int v)
 	return make_int2(w.x, w.y);
 }
 
-// Consumer side of DIRECT (FP16/BF16 storage): the views staged in LDS
-// first, in view order, then -- after the stage's LDS views, which only
-// changes the FP32 summation order -- any view whose footprint exceeded the
-// slot, gathered from HBM.  Keeping the two apart keeps one code path over
-// the accumulators in the main loop, so they stay in place in registers.
+// Consumer side of DIRECT (FP16/BF16 storage): the stage's views from view v on
+// that are staged in LDS, then the run of views behind them whose footprints
+// exceeded the slot, gathered from HBM; returns the view to go on with (nv: the
+// stage is done).  The order of additions is thus that of the views whatever the
+// slot and the views per stage, and an axial scan's bits depend on neither.
+// Keeping the two apart keeps one code path over the accumulators in the main
+// loop, so they stay in place in registers; the caller's one loop over stages and
+// runs does too (a loop over the runs in here spills 170 registers).
 // Every slice of a group a wave works on inside the view's slice window is
 // computed with u clamped to [0, u_hi] (ColRange): slices outside a lane's
 // range read zero rows with vertical weight 0, and lanes without work read
@@ -1029,14 +1032,17 @@ __device__ __forceinline__ int2 view_window(const BackArgs &a, int v)
 // z-group, ZL slices each, with accumulators accs[r]; one pass over the
 // stage's views adds all of them (each view's record and window read once).
 template <int NCW, int R, int ZL, int FMT, bool WINDOW>
-__device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
-	const Lds<NCW * R, false> &L, int v0, int nv, int wave, int lane, int zg0,
+__device__ __forceinline__ int consume_direct(const BackArgs &a, int bo,
+	const Lds<NCW * R, false> &L, int v0, int v, int nv, int wave, int lane, int zg0,
 	float (&accs)[R][ZL])
 {
 	const GeomF &g = a.g;
+	// the lane's record addresses are made anew for each run: kept over the stages
+	// they would be spilled, and each stage begin with two loads from scratch
+	// (clinical_arc FP16 7.88 ms for 7.70)
+	asm volatile("" : "+v"(lane));
 	const float4 *P4 = reinterpret_cast<const float4 *>(fdk_lds + bo + L.P) + lane;
 	const float2 *Q2 = reinterpret_cast<const float2 *>(fdk_lds + bo + L.Q) + lane;
-	const int2 *VI = reinterpret_cast<const int2 *>(fdk_lds + bo + L.vinfo + 2);
 	const int *ZR = reinterpret_cast<const int *>(fdk_lds + bo + L.vinfo);
 	const float za = anchor_z(g, !WINDOW, zg0);
 	// relative to the z-group: chunk r starts at slice zoff(r)
@@ -1052,16 +1058,9 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 		const int zc = zg0 + zoff(r);
 		return WINDOW ? make_int2(max(wa.x - zc, 0), min(wa.y - zc, ZL)) : make_int2(0, ZL);
 	};
-	bool hbm_views = false, cut_views = false;
-	int nzr = ZR[0];
-	for (int vv = 0; vv < nv; ++vv) {
-		const int zr = __builtin_amdgcn_readfirstlane(nzr);
-		if (vv + 1 < nv)
-			nzr = ZR[(vv + 1) * 4];
-		const int mode = zr & 3;
-		hbm_views = hbm_views || mode == MODE_GLOBAL;
-		if (mode != MODE_LDS)
-			continue;
+	bool cut_views = false;
+	// adds staged view vv; zr: the first word of its header
+	auto add_staged = [&](int vv, int zr) {
 		// the union of the tile's slice ranges (scalar): a group inside it
 		// where some lanes have no slices adds exactly 0 for those lanes
 		const int ulo = (zr >> 2) & 1023, uhi = (zr >> 12) & 1023;
@@ -1070,7 +1069,7 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 		for (int r = 0; r < R; ++r)
 			meets = meets || (ulo < zoff(r) + ZL && uhi > zoff(r));
 		if (!meets)
-			continue;                  // no lane of this wave meets the view
+			return;                    // no lane of this wave meets the view
 		const float4 p0 = P4[vv * 64];
 		const int c1 = bo + __float_as_int(p0.x);
 		const float wl = p0.y, wr = p0.z;
@@ -1131,64 +1130,11 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 				}
 			}
 		}
-	}
-	if (cut_views) {
-		// groups of 8 slices that a view's window cuts: the slices outside the
-		// window keep their sums (a select on a wave-uniform condition)
-		for (int vv = 0; vv < nv; ++vv) {
-			const int zr = __builtin_amdgcn_readfirstlane(ZR[vv * 4]);
-			if ((zr & 3) != MODE_LDS)
-				continue;
-			const int2 wa = view_window<WINDOW>(a, v0 + vv);
-			bool cut = false;
-#pragma unroll
-			for (int r = 0; r < R; ++r) {
-				const int2 w = window(wa, r);
-				cut = cut || !(w.x <= 0 && w.y >= ZL);
-			}
-			if (!cut)
-				continue;
-			const int ulo = (zr >> 2) & 1023, uhi = (zr >> 12) & 1023;
-			const float4 p0 = P4[vv * 64];
-			const int c1 = bo + __float_as_int(p0.x);
-			const float wl = p0.y, wr = p0.z;
-			const float2 q2 = Q2[vv * 64];
-		const float ti = q2.x, uh = q2.y;
-#pragma unroll
-			for (int r = 0; r < R; ++r) {
-				float (&acc)[ZL] = accs[r];
-				const int jlo = max(ulo - zoff(r), 0);
-				const int jhi = min(uhi - zoff(r), ZL);
-				const int2 w = window(wa, r);
-				if (jlo >= jhi || (w.x <= 0 && w.y >= ZL))
-					continue;
-#pragma unroll
-				for (int g0 = 0; g0 < ZL; g0 += 8) {
-					if (g0 >= w.y || g0 + 8 <= w.x || (w.x <= g0 && g0 + 8 <= w.y)
-						|| g0 >= jhi || g0 + 8 <= jlo)
-						continue;
-					const float t8 = u8(r, g0, ti, p0.w);
-#pragma unroll
-					for (int j = g0; j < g0 + 8; ++j) {
-						const float u = __builtin_amdgcn_fmed3f(fmaf((float) (j - g0), ti, t8),
-							0.f, uh);
-						const float up = slice_update_d<FMT>(acc[j], u, c1, wl, wr);
-						acc[j] = (j >= w.x && j < w.y) ? up : acc[j];
-					}
-				}
-			}
-		}
-	}
-	if (!hbm_views)
-		return;
-	// views whose footprint exceeded the LDS slot: gather from the caller's
-	// views, zero outside the detector; lanes without work in a view read
-	// columns left of the detector (zeros)
-	for (int vv = 0; vv < nv; ++vv) {
-		const int2 vi = VI[vv * 2];
-		if ((__builtin_amdgcn_readfirstlane(vi.y) >> 16) != MODE_GLOBAL)
-			continue;
-		const int zr = __builtin_amdgcn_readfirstlane(ZR[vv * 4]);
+	};
+	// adds view vv, whose footprint exceeded the slot, from the caller's views, zero
+	// outside the detector; lanes without work in it read columns left of the
+	// detector (zeros)
+	auto add_gathered = [&](int vv, int zr) {
 		const int ulo = (zr >> 2) & 1023, uhi = (zr >> 12) & 1023;
 		const float4 p0 = P4[vv * 64];
 		const float wl = p0.y, wr = p0.z;
@@ -1220,7 +1166,69 @@ __device__ __forceinline__ void consume_direct(const BackArgs &a, int bo,
 				__builtin_amdgcn_sched_barrier(0);
 			}
 		}
+	};
+	// the stage's headers, view i's in lane i (a stage has at most 64 views); from
+	// them the staged views [v, vl) and the gathered ones behind them [vl, vg)
+	const int hdr = ZR[min(lane, nv - 1) * 4];
+	const unsigned long long m = __ballot(lane < nv && (hdr & 3) == MODE_GLOBAL) >> v;
+	const unsigned long long past = m ? ~(m >> __builtin_ctzll(m)) : 0;
+	const int vl = m ? v + __builtin_ctzll(m) : nv;
+	const int vg = past ? min(vl + __builtin_ctzll(past), nv) : nv;
+	for (int vv = v; vv < vl; ++vv) {
+		const int zr = __builtin_amdgcn_readlane(hdr, vv);
+		if ((zr & 3) == MODE_LDS)
+			add_staged(vv, zr);
 	}
+	if (cut_views) {
+		// groups of 8 slices that a view's window cuts: the slices outside the
+		// window keep their sums (a select on a wave-uniform condition)
+		for (int vv = v; vv < vl; ++vv) {
+			const int zr = __builtin_amdgcn_readlane(hdr, vv);
+			if ((zr & 3) != MODE_LDS)
+				continue;
+			const int2 wa = view_window<WINDOW>(a, v0 + vv);
+			bool cut = false;
+#pragma unroll
+			for (int r = 0; r < R; ++r) {
+				const int2 w = window(wa, r);
+				cut = cut || !(w.x <= 0 && w.y >= ZL);
+			}
+			if (!cut)
+				continue;
+			const int ulo = (zr >> 2) & 1023, uhi = (zr >> 12) & 1023;
+			const float4 p0 = P4[vv * 64];
+			const int c1 = bo + __float_as_int(p0.x);
+			const float wl = p0.y, wr = p0.z;
+			const float2 q2 = Q2[vv * 64];
+			const float ti = q2.x, uh = q2.y;
+#pragma unroll
+			for (int r = 0; r < R; ++r) {
+				float (&acc)[ZL] = accs[r];
+				const int jlo = max(ulo - zoff(r), 0);
+				const int jhi = min(uhi - zoff(r), ZL);
+				const int2 w = window(wa, r);
+				if (jlo >= jhi || (w.x <= 0 && w.y >= ZL))
+					continue;
+#pragma unroll
+				for (int g0 = 0; g0 < ZL; g0 += 8) {
+					if (g0 >= w.y || g0 + 8 <= w.x || (w.x <= g0 && g0 + 8 <= w.y)
+						|| g0 >= jhi || g0 + 8 <= jlo)
+						continue;
+					const float t8 = u8(r, g0, ti, p0.w);
+#pragma unroll
+					for (int j = g0; j < g0 + 8; ++j) {
+						const float u = __builtin_amdgcn_fmed3f(fmaf((float) (j - g0), ti, t8),
+							0.f, uh);
+						const float up = slice_update_d<FMT>(acc[j], u, c1, wl, wr);
+						acc[j] = (j >= w.x && j < w.y) ? up : acc[j];
+					}
+				}
+			}
+		}
+	}
+	for (int vv = vl; vv < vg; ++vv)
+		add_gathered(vv, __builtin_amdgcn_readlane(hdr, vv));
+	return vg;
 }
 
 // Workgroup = NW consumer waves (z chunks of ZL slices, lane = column) and
@@ -1287,18 +1295,23 @@ __device__ __forceinline__ void tile_pipeline(const BackArgs &a, int tile, int g
 			for (int j = 0; j < ZL; ++j)
 				accs[r][j] = 0.f;
 		__syncthreads();
-		for (int s = 0; s < nstage; ++s) {
-			const int v0 = va + s * a.vstage;
-			if constexpr (FMT == FMT_F32)
-				consume_walk<NW, R, ZL, FMT, FAST>(a, (s & 1) * L.total, L, v0,
-					min(a.vstage, vb - v0), wave, lane, zg0, accs);
-			else {
+		for (int s = 0, v = 0; s < nstage;) {   // v: the stage's next view
+			const int v0 = va + s * a.vstage, nv = min(a.vstage, vb - v0);
+			if constexpr (FMT == FMT_F32) {
+				consume_walk<NW, R, ZL, FMT, FAST>(a, (s & 1) * L.total, L, v0, nv, wave, lane,
+					zg0, accs);
+				v = nv;
+			} else {
 				// chunks wave + r NW of the z-group in one pass over the
 				// stage's views (u is in closed form from the group's U0)
-				consume_direct<NW, R, ZL, FMT, WIN>(a, (s & 1) * L.total, L, v0,
-					min(a.vstage, vb - v0), wave, lane, zg0, accs);
+				v = consume_direct<NW, R, ZL, FMT, WIN>(a, (s & 1) * L.total, L, v0, v, nv, wave,
+					lane, zg0, accs);
 			}
-			__syncthreads();
+			if (v == nv) {
+				__syncthreads();
+				v = 0;
+				++s;
+			}
 		}
 		// one write per voxel, [nz nx ny]
 		if (ix < g.nx && iy < g.ny) {

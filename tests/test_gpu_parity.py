@@ -280,6 +280,32 @@ def test_16bit_row_coordinate_rounding(device, dz, fmt):
 
 
 @pytest.mark.parametrize("fmt", ["f16", "bf16"])
+@pytest.mark.parametrize("ds,ns", [(3.0, 40), (0.7, 180)])
+def test_16bit_bits_do_not_depend_on_slot(device, ds, ns, fmt):
+    """Footprints of about 6 and 28 columns per 8 x 8 tile in slots that hold
+    all, some and none of them, with 1 to 19 views per stage: gathered and
+    staged views are added in view order with the same arithmetic, so the bits
+    are those of the launch whose slots hold every footprint."""
+    import torch
+    from mirt_amd import quantize_views
+    g = O.geom((41, 38, 150), (2.0, -2.0, 1.0), (0.25, 0.0, -0.5), 541.0, 949.0, 0.0,
+               ns, 37, (ds, 4.3), (0.25, 0.0))
+    proj = np.random.default_rng(ns).standard_normal((19, ns, 37)).astype(np.float32)
+    beta = np.linspace(0, 6, 19)
+    mask = np.ones((38, 41), np.uint8)
+    q, sc = quantize_views(torch.from_numpy(proj).to(device), fmt)
+    plan = _plan(g, beta, mask, fmt)
+    img = [plan(q, sc).cpu().numpy()]
+    for waves, zper, vstage, cap in ((4, 8, 2, 0), (4, 8, 2, 64), (4, 8, 19, 192), (8, 16, 3, 128),
+                                     (4, 48, 5, 256), (4, 48, 1, 64), (4, 16, 4, 320),
+                                     (4, 32, 3, 192), (8, 32, 2, 256), (4, 64, 3, 128)):
+        plan.set_config(waves, zper, vstage, cap)
+        img.append(plan(q, sc).cpu().numpy())
+        assert np.array_equal(img[-1], img[0]), (waves, zper, vstage, cap)
+    assert np.any(img[0])
+
+
+@pytest.mark.parametrize("fmt", ["f16", "bf16"])
 def test_occupancy_builds_same_bits(device, fmt):
     """The 8-waves-per-SIMD kernel build of one-chunk FP16/BF16 shapes gives
     the same bits as the 4-wave build (same instructions, other register
