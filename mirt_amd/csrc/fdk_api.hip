@@ -256,18 +256,39 @@ static BackArgs make_args(const fdkhip_plan *p, const void *proj, const float *s
 	return a;
 }
 
+// `device` as the current device while the object lives
+class DeviceScope {
+	int before = -1;   // to go back to
+	hipError_t err;
+
+public:
+	explicit DeviceScope(int device)
+	{
+		int cur = 0;
+		err = hipGetDevice(&cur);
+		if (err == hipSuccess && cur != device) {
+			err = hipSetDevice(device);
+			if (err == hipSuccess)
+				before = cur;
+		}
+	}
+	~DeviceScope()
+	{
+		if (before >= 0)
+			(void) hipSetDevice(before);
+	}
+	DeviceScope(const DeviceScope &) = delete;
+	DeviceScope &operator=(const DeviceScope &) = delete;
+	hipError_t error() const { return err; }
+};
+
 // Waits for all work on `device`: a batch's graph exec or a buffer about to be
 // destroyed may still be in use by a launch queued on any stream.
 static void quiesce(int device)
 {
-	int cur = 0;
-	if (hipGetDevice(&cur) != hipSuccess)
-		return;
-	if (cur != device)
-		(void) hipSetDevice(device);
-	(void) hipDeviceSynchronize();
-	if (cur != device)
-		(void) hipSetDevice(cur);
+	const DeviceScope scope(device);
+	if (scope.error() == hipSuccess)
+		(void) hipDeviceSynchronize();
 }
 
 // Stage depth (views per LDS stage) and slot size (floats per staged view)
@@ -561,13 +582,14 @@ static int set_tiling(fdkhip_plan *p, int nw, int zper)
 	return FDKHIP_OK;
 }
 
-// The exact survey of the current tiling (cached per tiling): the reference's
-// loop iterations, the largest footprint, whether any column meets any view.
-static int run_survey(fdkhip_plan *p)
+// The exact survey of the current tiling (cached per tiling) on stream `ss`: the
+// reference's loop iterations, the largest footprint, whether any column meets
+// any view.  After a failure the count is unknown.
+static int run_survey(fdkhip_plan *p, hipStream_t ss)
 {
 	p->maxarea = 0;
 	p->fov_any = 0;
-	p->n_updates = 0;
+	p->n_updates = -1;
 	for (const auto &sv : p->surveys)
 		if (sv.nw == p->nw && sv.zl == p->zl && sv.zr == p->zr) {
 			p->maxarea = sv.maxarea;
@@ -575,9 +597,12 @@ static int run_survey(fdkhip_plan *p)
 			p->n_updates = sv.n_updates;
 			return FDKHIP_OK;
 		}
-	if (p->ngroups == 0 || p->tiles_x == 0 || p->tiles_y == 0 || p->na == 0)
+	if (p->ngroups == 0 || p->tiles_x == 0 || p->tiles_y == 0 || p->na == 0) {
+		p->n_updates = 0;
 		return FDKHIP_OK;
-	hipStream_t ss = p->survey_stream;
+	}
+	const DeviceScope scope(p->device);   // the plan's, whichever is current
+	HIP_TRY(scope.error());
 	HIP_TRY(launch_zero_u64(p->d_count, 1, ss));
 	HIP_TRY(launch_zero_i32(p->d_maxarea, 1, ss));
 	HIP_TRY(launch_zero_i32(p->d_any, 1, ss));
@@ -600,7 +625,7 @@ static int configure(fdkhip_plan *p, int nw, int zper, int vstage_req, int slot_
 {
 	int rc = set_tiling(p, nw, zper);
 	if (!rc)
-		rc = run_survey(p);
+		rc = run_survey(p, p->survey_stream);
 	if (rc)
 		return rc;
 	int vstage = 0, slot = 0;
@@ -637,7 +662,7 @@ static int check_direction(fdkhip_plan *p)
 {
 	if (p->gf.dz / p->gf.dt >= 0)
 		return FDKHIP_OK;
-	const int rc = run_survey(p);
+	const int rc = run_survey(p, p->survey_stream);
 	if (rc || !p->fov_any)
 		return rc;
 	return fail(FDKHIP_EGEOM, "todo: dz/dt < 0 not done");
@@ -844,7 +869,19 @@ extern "C" int fdkhip_plan_count_updates(fdkhip_plan *p, int64_t *n)
 	if (!p || !n)
 		return fail(FDKHIP_EARG, "NULL argument");
 	if (p->n_updates < 0) {
-		const int rc = run_survey(p);
+		// a plan whose launch shape needed no survey: counted now, on a stream of
+		// its own that a capture under way on this thread does not see
+		const DeviceScope scope(p->device);
+		HIP_TRY(scope.error());
+		hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+		HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+		hipStream_t ss = nullptr;
+		const hipError_t e = hipStreamCreateWithFlags(&ss, hipStreamNonBlocking);
+		const int rc = e == hipSuccess ? run_survey(p, ss)
+			: fail(FDKHIP_EHIP, "hipStreamCreateWithFlags: %s", hipGetErrorString(e));
+		if (ss)
+			(void) hipStreamDestroy(ss);
+		(void) hipThreadExchangeStreamCaptureMode(&mode);
 		if (rc)
 			return rc;
 	}

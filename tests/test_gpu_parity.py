@@ -455,3 +455,25 @@ def test_direct_hbm_gather_path(device, fmt):
             err = O.rel_l2(img, O.back_ts_f64(g, _stored(q, sc), beta, mask))
             print(f"  relL2 = {err:.3e}", flush=True)
             assert err <= 1e-5, err
+
+
+def test_count_updates_under_capture(device):
+    """The count of an untuned plan is taken on demand; asked for while the
+    thread captures a graph, it is the number of the same plan outside, and the
+    capture goes on."""
+    import torch
+    g, proj, beta, mask = make_case("arc", seed=4)
+    p = torch.from_numpy(proj).to(device)
+    want = _plan(g, beta, mask).count_updates()
+    plan = _plan(g, beta, mask)
+    out = torch.empty((g.ny, g.nx, g.nz), device=device)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        n = plan.count_updates()
+        plan(p, out=out)
+    assert n == want > 0
+    for rep in range(3):
+        out.fill_(rep)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), O.back_ts_f32(g, proj, beta, mask)), rep

@@ -1,0 +1,92 @@
+"""Host code of the library against a stand-in HIP runtime (tests/hip_stub).
+
+Each test runs in a process of its own (no GPU, no torch): the stand-in is
+loaded first with RTLD_GLOBAL, so that libfdkhip.so's HIP calls come to it; it
+logs launches and copies, keeps device memory on the host and lets chosen
+calls fail.  Kernels do not run, so only what the host decides is tested:
+devices, launch grids, layouts, error paths.
+"""
+from __future__ import annotations
+
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+from conftest import ROOT
+
+STUB = os.path.join(ROOT, "tests", "hip_stub", "fake_hip.c")
+
+PREAMBLE = """
+import ctypes as C, sys, time
+sys.path.insert(0, %(root)r)
+fake = C.CDLL(%(stub)r, mode=C.RTLD_GLOBAL)
+fake.fake_log.restype = C.c_char_p
+fake.fake_fail.argtypes = [C.c_char_p, C.c_int]
+fake.fake_fast_lds.argtypes = [C.c_size_t]
+import numpy as np
+from mirt_amd import _lib
+lib = _lib.load()
+F32, F16 = _lib.F32, _lib.F16
+
+def log(kind=None):
+    rows = [r.split() for r in fake.fake_log().decode().splitlines()]
+    return [[int(x) for x in r[1:]] for r in rows if r[0] == kind] if kind else rows
+
+def geom(nx, ny, nz, ns, nt, dx=1.0, dz=1.0, ds=1.0, dt=1.0):
+    return _lib.Geom(nx, ny, nz, dx, -dx, dz, 0, 0, 0, 541.0, 949.0, float("inf"), ns, nt,
+                     ds, dt, 0, 0)
+
+def plan(g, na=24, fmt=F32):
+    h, beta = C.c_void_p(), np.linspace(0, 6, na)
+    _lib.check(lib.fdkhip_plan_create(C.byref(h), C.byref(g), na,
+                                      C.c_void_p(beta.ctypes.data), None, fmt, 0))
+    return h
+
+BUF = C.c_void_p(1 << 20)   # a device buffer that no kernel reads
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("hip_stub") / "libfakehip.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-I/opt/rocm/include", "-o", out, STUB],
+                   check=True)
+    return out
+
+
+def _run(stub, body):
+    code = PREAMBLE % dict(root=ROOT, stub=stub) + textwrap.dedent(body) + "\nprint('passed')\n"
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.endswith("passed\n"), r.stdout + r.stderr
+
+
+def test_count_updates_device_and_failures(stub):
+    """The count of a plan whose shape needed no survey runs on the plan's own
+    device and stream whichever device is current, goes back to that device,
+    and stays unknown after a failure."""
+    _run(stub, """
+    fake.fake_fill(1)
+    for fmt in (F32, F16):
+        h, n = plan(geom(64, 64, 32, 128, 96), fmt=fmt), C.c_int64(-7)
+        assert not log("launch")          # no survey
+        fake.hipSetDevice(1)
+        fake.fake_fail(b"hipStreamSynchronize", 1)
+        assert lib.fdkhip_plan_count_updates(h, C.byref(n)) == -4 and n.value == -7
+        fake.fake_clear()
+        assert lib.fdkhip_plan_count_updates(h, C.byref(n)) == 0
+        assert n.value == 0x0101010101010101
+        rows = log("launch")
+        assert rows and all(r[0] == 0 and r[-1] != 0 for r in rows), rows
+        assert all(r[0] == 0 for r in log("memcpy"))
+        d = C.c_int()
+        fake.hipGetDevice(C.byref(d))
+        assert d.value == 1
+        fake.fake_clear()
+        assert lib.fdkhip_plan_count_updates(h, C.byref(n)) == 0 and not log()
+        fake.hipSetDevice(0)
+        lib.fdkhip_plan_destroy(h)
+        fake.fake_clear()
+    """)
