@@ -50,7 +50,6 @@ struct EllArgs {
 	int ns, nt, na, nell, no;        // no: oversampling factor
 	double ds, dt, dso, dod;         // sample spacing (oversampling), distances
 	int kind;
-	unsigned nblk;                   // workgroups per block of views
 	double *proj;                    // [na][nt][ns]
 };
 
@@ -117,9 +116,9 @@ ellipsoid_proj_kernel(const EllArgs a)
 		E[k] = a.ell[k];
 	__syncthreads();
 	const long nst = (long) a.ns * a.nt;
-	const unsigned vb = blockIdx.x / a.nblk;   // view block, block of samples
-	const long i = (long) (blockIdx.x - vb * a.nblk) * blockDim.x + threadIdx.x;
-	if (i >= nst)
+	const long i = (long) blockIdx.x * blockDim.x + threadIdx.x;
+	const long vb = (long) blockIdx.z * gridDim.y + blockIdx.y;   // block of views
+	if (i >= nst || vb * ELL_VIEWS >= a.na)
 		return;
 	const int is = (int) (i % a.ns), it = (int) (i / a.ns);
 	const int v0 = (int) vb * ELL_VIEWS;
@@ -290,11 +289,12 @@ extern "C" int fdkhip_ellipsoid_proj(const double *s, int32_t ns, const double *
 		a.kind = kind;
 		a.proj = proj_dev;
 		const long nst = (long) ns * nt;
-		a.nblk = (unsigned) ((nst + 255) / 256);
-		const long blocks = (long) a.nblk * ((na + ELL_VIEWS - 1) / ELL_VIEWS);
-		ELL_TRY(blocks > 0x7fffffffL ? hipErrorInvalidValue : hipSuccess);
-		hipLaunchKernelGGL(ellipsoid_proj_kernel, dim3((unsigned) blocks), dim3(256),
-			nrow * sizeof(EllRow), st, a);
+		// samples along x, blocks of views along y and z: a grid has less than 2^32
+		// threads along a dimension and at most 65535 workgroups along y and z
+		const long vblocks = ((long) na + ELL_VIEWS - 1) / ELL_VIEWS;
+		const unsigned gy = (unsigned) std::min(vblocks, 65535L);
+		const dim3 grid((unsigned) ((nst + 255) / 256), gy, (unsigned) ((vblocks + gy - 1) / gy));
+		hipLaunchKernelGGL(ellipsoid_proj_kernel, grid, dim3(256), nrow * sizeof(EllRow), st, a);
 		ELL_TRY(hipGetLastError());
 		// the host table above is released at return: wait for the copy
 		ELL_TRY(hipStreamSynchronize(st));

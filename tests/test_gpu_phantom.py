@@ -79,3 +79,35 @@ def test_ellipsoid_kernel_views_and_errors(device):
     odd = ct_geom("fan", ns=8, nt=4, na=2, ds=1.0, dt=1.0, dsd=949.0, dso=541.0, dfs=100.0)
     with pytest.raises(FdkhipError, match="not done"):
         ellipsoid_proj(odd, ell, device=device)
+
+
+def test_ellipsoid_kernel_many_views(device):
+    """More blocks of views than a grid has along y: the first, middle and last
+    views are those of a call that takes them alone, bit for bit (the same
+    kernel and table entries)."""
+    from mirt_amd.geom import ct_geom
+    from mirt_amd.phantom import ellipsoid_proj
+    na = 4 * 65535 + 9
+    cg = ct_geom("fan", ns=3, nt=2, na=na, ds=20.0, dt=15.0, dsd=949.0, dso=541.0, dfs=0.0)
+    ell = _phantom(33, n=4)
+    got = ellipsoid_proj(cg, ell, device=device)
+    for views in ([0, 1, 2, 3, 4, 5], [4 * 65535 - 1, 4 * 65535, 4 * 65535 + 1], [na - 2, na - 1]):
+        want = ellipsoid_proj(cg, ell, device=device, views=views).cpu().numpy()
+        assert np.any(want) and np.array_equal(got[:, :, views].cpu().numpy(), want), views
+
+
+@pytest.mark.parametrize("scale", [1e-120, 1e-50, 1e90])
+def test_ellipsoid_kernel_scaled_geometry(device, scale):
+    """Lengths far from 1 take the chord's library root and quotient where the
+    product under the root leaves 1e+-280: the same geometry scaled gives
+    scaled line integrals, to the bar of this file."""
+    from mirt_amd.geom import ct_geom
+    from mirt_amd.phantom import ellipsoid_proj
+    ell = np.array([[3.0, -2.0, 1.0, 10.0, 14.0, 12.0, 25.0, 0, 0.5],
+                    [-4.0, 5.0, 0.5, 6.0, 3.0, 9.0, 70.0, 0, 0.2]])
+    big = ell.copy()
+    big[:, :6] *= scale
+    kw = dict(ns=41, nt=9, na=5)
+    want = ellipsoid_proj(ct_geom("fan", ds=1.0, dt=1.0, dsd=np.inf, **kw), ell, device=device)
+    got = ellipsoid_proj(ct_geom("fan", ds=scale, dt=scale, dsd=np.inf, **kw), big, device=device)
+    assert _rel(got.cpu().numpy() / scale, want.cpu().numpy()) <= 1e-10

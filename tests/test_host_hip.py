@@ -90,3 +90,20 @@ def test_count_updates_device_and_failures(stub):
         lib.fdkhip_plan_destroy(h)
         fake.fake_clear()
     """)
+
+
+@pytest.mark.parametrize("ns,nt,na", [(4096, 4096, 2000), (2, 1, 262145), (3, 5, 1)])
+def test_phantom_grid(stub, ns, nt, na):
+    """The phantom's grid covers every sample and view within a grid's limits:
+    less than 2^32 threads along a dimension, 65535 workgroups along y and z."""
+    _run(stub, f"""
+    ns, nt, na = {ns}, {nt}, {na}
+    s, t, b = np.arange(ns, dtype=float), np.arange(nt, dtype=float), np.linspace(0, 6, na)
+    ell = np.array([[0, 0, 0, 10, 10, 10, 0, 0, 0.5]], float)
+    P = lambda a: C.c_void_p(a.ctypes.data)
+    _lib.check(lib.fdkhip_ellipsoid_proj(P(s), ns, P(t), nt, P(b), None, na, 541.0, 408.0, 0.0,
+                                         P(ell), 1, 1, BUF, None))
+    [(dev, gx, gy, gz, threads, lds, st)] = log("launch")
+    assert gx * threads >= ns * nt and gx * threads < 2 ** 32, (gx, threads)
+    assert gy <= 65535 and gz <= 65535 and gy * gz * 4 >= na, (gy, gz)
+    """)
