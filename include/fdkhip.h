@@ -314,10 +314,11 @@ int fdkhip_plan_destroy(fdkhip_plan *plan);
  * computed on the device.  Synchronous. */
 int fdkhip_plan_count_updates(fdkhip_plan *plan, int64_t *n_updates);
 
-/* Time every launch shape the build supports with each views-per-stage depth
- * that fits LDS and each kernel build (`reps` launches of the backprojection
- * kernel each, over the first 128 views, on `stream`), time the four fastest
- * again over all views (plans of more than 128 views), keep the fastest for
+/* Time the plan's untuned layout and every launch shape the build supports with
+ * each views-per-stage depth that fits LDS, in each kernel build (`reps`
+ * launches of the backprojection kernel each, over the first 128 views, on
+ * `stream`), time the four fastest and the untuned one again over all views
+ * (plans of more than 128 views), keep the fastest for
  * this plan and remember it for later plans of the same geometry, view
  * count, format and math mode in this process.  image_dev is overwritten
  * (its contents are undefined afterwards).  *best_ms (may be NULL) receives

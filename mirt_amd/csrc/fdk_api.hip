@@ -2164,6 +2164,7 @@ const int kTuneFinalists = 4; // fastest candidates timed again over all views
 struct Tuned {
 	int nw, zl, vstage;   // zl: slices per consumer wave (the configuration's zper)
 	int minw = 4;         // kernel build: minimum waves per SIMD
+	int slot = 0;         // LDS slot, where it is the untuned layout's; 0: by the survey
 };
 
 std::mutex g_tune_mu;
@@ -2235,6 +2236,20 @@ static int time_launches(const std::function<int(hipStream_t)> &run, hipStream_t
 	return rc;
 }
 
+// A layout as the tuner keeps it: with a slot of its own, or one by the survey.
+static int apply_layout(fdkhip_plan *p, const Tuned &t)
+{
+	p->minw = t.minw;
+	if (t.slot == 0)
+		return configure(p, t.nw, t.zl, t.vstage, 0);
+	const int rc = set_tiling(p, t.nw, t.zl);
+	if (rc)
+		return rc;
+	p->vstage = t.vstage;
+	p->slot = t.slot;
+	return FDKHIP_OK;
+}
+
 extern "C" int fdkhip_plan_autotune(fdkhip_plan *p, const void *proj, const float *scale,
 	float *image, void *stream, int32_t reps, float *best_ms)
 {
@@ -2244,7 +2259,7 @@ extern "C" int fdkhip_plan_autotune(fdkhip_plan *p, const void *proj, const floa
 	if (reps < 1)
 		return fail(FDKHIP_EARG, "reps must be >= 1");
 	hipStream_t s = (hipStream_t) stream;
-	Tuned best{p->nw, p->zl * p->zr, p->vstage, plan_minw(p)};
+	Tuned best{p->nw, p->zl * p->zr, p->vstage, plan_minw(p), p->slot};
 	float best_t = 3.4e38f;
 	// the padded views once; then the backprojection kernel alone over the
 	// first kTuneViews views (its time is proportional to the view count)
@@ -2252,6 +2267,43 @@ extern "C" int fdkhip_plan_autotune(fdkhip_plan *p, const void *proj, const floa
 	if (rc)
 		return rc;
 	std::vector<std::pair<float, Tuned>> cand;
+	// times each kernel build that the plan's current shape has (4 waves per SIMD;
+	// 8 for one-chunk FP16/BF16 shapes)
+	auto time_builds = [&](Tuned t) {
+		if (p->ngroups == 0 || p->na == 0)
+			return FDKHIP_OK;
+		for (int mw : {4, 8}) {
+			if (!back_minw_supported(mw, p->zr, p->fmt))
+				continue;
+			p->minw = t.minw = mw;
+			float ms = 0.f;
+			const int rc = time_launches([&](hipStream_t st) {
+				BackArgs a = make_args(p, proj, scale, image);
+				a.g.na = std::min(p->na, kTuneViews);
+				HIP_TRY(launch_back(a, p->nw, p->zl, p->zr, p->fmt,
+					p->math == FDKHIP_MATH_FAST, plan_minw(p), st));
+				return FDKHIP_OK;
+			}, s, reps, &ms);
+			if (rc)
+				return rc;
+			cand.emplace_back(ms, t);
+			if (ms < best_t) {
+				best_t = ms;
+				best = t;
+			}
+		}
+		return FDKHIP_OK;
+	};
+	// the untuned layout, whose slots may be cut for residency, then every shape
+	// with slots that hold the largest footprint
+	if (p->def_vstage > 0) {
+		const Tuned t{p->def_nw, p->def_zper, p->def_vstage, 4, p->def_slot};
+		rc = apply_layout(p, t);
+		if (!rc)
+			rc = time_builds(t);
+		if (rc)
+			return rc;
+	}
 	for (const auto &sh : kPlanShapes) {
 		int last_vstage = -1;
 		for (int vs : kStages) {
@@ -2260,46 +2312,30 @@ extern "C" int fdkhip_plan_autotune(fdkhip_plan *p, const void *proj, const floa
 			if (p->vstage == last_vstage)
 				continue;   // the LDS budget clamped it to a depth already timed
 			last_vstage = p->vstage;
-			if (p->ngroups == 0 || p->na == 0)
-				continue;
-			// each kernel build this shape has (4 waves per SIMD; 8 for one-chunk
-			// FP16/BF16 shapes)
-			for (int mw : {4, 8}) {
-				if (!back_minw_supported(mw, p->zr, p->fmt))
-					continue;
-				p->minw = mw;
-				float t = 0.f;
-				rc = time_launches([&](hipStream_t st) {
-					BackArgs a = make_args(p, proj, scale, image);
-					a.g.na = std::min(p->na, kTuneViews);
-					HIP_TRY(launch_back(a, p->nw, p->zl, p->zr, p->fmt,
-						p->math == FDKHIP_MATH_FAST, plan_minw(p), st));
-					return FDKHIP_OK;
-				}, s, reps, &t);
-				if (rc)
-					return rc;
-				cand.emplace_back(t, Tuned{sh[0], sh[1], p->vstage, mw});
-				if (t < best_t) {
-					best_t = t;
-					best = Tuned{sh[0], sh[1], p->vstage, mw};
-				}
-			}
+			rc = time_builds(Tuned{sh[0], sh[1], p->vstage});
+			if (rc)
+				return rc;
 		}
 	}
 	if (p->na > kTuneViews && cand.size() > 1) {
-		// the fastest few again over all views: a prefix can rank shapes
-		// whose start-up and per-view costs differ in another order
+		// the fastest few, and the untuned layout, again over all views: a prefix
+		// can rank shapes whose start-up and per-view costs differ in another order
+		const std::pair<float, Tuned> untuned = cand.front();
 		std::sort(cand.begin(), cand.end(),
 			[](const std::pair<float, Tuned> &x, const std::pair<float, Tuned> &y) {
 				return x.first < y.first;
 			});
 		cand.resize(std::min(cand.size(), (size_t) kTuneFinalists));
+		if (untuned.second.slot > 0 && std::none_of(cand.begin(), cand.end(),
+				[&](const std::pair<float, Tuned> &x) {
+					return x.second.slot > 0 && x.second.minw == untuned.second.minw;
+				}))
+			cand.push_back(untuned);
 		best_t = 3.4e38f;
 		for (const auto &c : cand) {
-			rc = configure(p, c.second.nw, c.second.zl, c.second.vstage, 0);
+			rc = apply_layout(p, c.second);
 			if (rc)
 				return rc;
-			p->minw = c.second.minw;
 			float t = 0.f;
 			rc = time_launches([&](hipStream_t st) {
 				const BackArgs a = make_args(p, proj, scale, image);
@@ -2315,10 +2351,9 @@ extern "C" int fdkhip_plan_autotune(fdkhip_plan *p, const void *proj, const floa
 			}
 		}
 	}
-	rc = configure(p, best.nw, best.zl, best.vstage, 0);
+	rc = apply_layout(p, best);
 	if (rc)
 		return rc;
-	p->minw = best.minw;
 	tuned_store(tune_key(p), best);
 	if (best_ms)
 		*best_ms = best_t;
@@ -2361,26 +2396,14 @@ extern "C" int fdkhip_plan_profile(fdkhip_plan *p, const void *proj, const float
 	return rc;
 }
 
-
-// apply a choice made earlier in this process for the same geometry
 // a plan's own launch shape: the autotuner's choice made earlier in this
 // process for the same geometry, or the one chosen when the plan was made,
 // whose slot needs no survey
 static int plan_default_config(fdkhip_plan *p)
 {
-	Tuned t;
-	if (tuned_lookup(tune_key(p), t)) {
-		p->minw = t.minw;
-		return configure(p, t.nw, t.zl, t.vstage, 0);
-	}
-	if (p->def_vstage == 0)
-		return configure(p, p->def_nw, p->def_zper, 0, 0);
-	const int rc = set_tiling(p, p->def_nw, p->def_zper);
-	if (rc)
-		return rc;
-	p->vstage = p->def_vstage;
-	p->slot = p->def_slot;
-	return FDKHIP_OK;
+	Tuned t{p->def_nw, p->def_zper, p->def_vstage, p->minw, p->def_slot};
+	(void) tuned_lookup(tune_key(p), t);
+	return apply_layout(p, t);
 }
 
 // ---------------------------------------------------------------------------

@@ -107,3 +107,27 @@ def test_phantom_grid(stub, ns, nt, na):
     assert gx * threads >= ns * nt and gx * threads < 2 ** 32, (gx, threads)
     assert gy <= 65535 and gz <= 65535 and gy * gz * 4 >= na, (gy, gz)
     """)
+
+
+@pytest.mark.parametrize("fmt", ["F32", "F16"])
+@pytest.mark.parametrize("na", [24, 200])
+def test_autotune_times_the_untuned_layout(stub, na, fmt):
+    """The tuner times the layout of the untuned plan too, in both of its rounds:
+    where that is the fastest (the only one the stand-in's clock gives 1 ms) the
+    plan keeps it, slot included, and so do later plans of the geometry."""
+    _run(stub, f"""
+    def layout(h):
+        fake.fake_clear()
+        _lib.check(lib.fdkhip_plan_execute(h, BUF, BUF, BUF, None))
+        cfg = (C.c_int32 * 6)()
+        _lib.check(lib.fdkhip_plan_config(h, cfg))
+        return list(cfg), log("launch")[-1]
+    h = plan(geom(256, 256, 128, 512, 384, 0.5, 0.5, 0.8, 0.8), {na}, {fmt})
+    want = layout(h)
+    fake.fake_fast_lds(want[1][5])
+    ms = C.c_float()
+    _lib.check(lib.fdkhip_plan_autotune(h, BUF, BUF, BUF, None, 1, C.byref(ms)))
+    assert ms.value == 1.0
+    assert layout(h) == want
+    assert layout(plan(geom(256, 256, 128, 512, 384, 0.5, 0.5, 0.8, 0.8), {na}, {fmt})) == want
+    """)
