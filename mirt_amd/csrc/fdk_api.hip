@@ -356,11 +356,13 @@ struct HeightSample {
 	std::vector<int> area;
 };
 
-constexpr int kSampleViews = 12, kSampleTiles = 7;
+constexpr int kSampleViews = 12, kSampleTiles = 7, kSampleGroups = 32;
 
 // Footprints as the backprojection kernel stages them, from the four corner
 // columns of at most kSampleTiles^2 tiles in kSampleViews views (their own
-// samples are the extremes of a tile's).  An estimate: a view whose footprint
+// samples are the extremes of a tile's), in at most kSampleGroups z-groups of a
+// height, so that the time does not grow with the slices (0.1 to 0.3 ms; over all
+// groups 16 ms for 20000 slices).  An estimate: a view whose footprint
 // turns out larger than its slot gathers from memory, added in its turn with the
 // same bits (an FP16/BF16 helix: with sums in another order, see consume_direct).
 static void sample_heights(const fdkhip_plan *p, const double *beta, const uint8_t *mask,
@@ -399,8 +401,11 @@ static void sample_heights(const fdkhip_plan *p, const double *beta, const uint8
 				smax = std::max(smax, s);
 			}
 			const double s0 = std::max(floor(smin) + 1, 0.), s1 = std::min(floor(smax) + 2, g.ns + 1.);
-			for (auto &h : hs)
-				for (int z0 = p->zs_lo; z0 < p->zs_hi; z0 += h.height) {
+			for (auto &h : hs) {
+				const int groups = (p->zs_hi - p->zs_lo + h.height - 1) / h.height;
+				const int ng = std::min(groups, kSampleGroups);
+				for (int k = 0; k < ng; ++k) {
+					const int z0 = p->zs_lo + h.height * (int) ((2L * k + 1) * groups / (2 * ng));
 					++h.groups;
 					if (!ok || s0 > s1)
 						continue;
@@ -422,6 +427,7 @@ static void sample_heights(const fdkhip_plan *p, const double *beta, const uint8
 					h.area.push_back((int) std::min(a, 0x7fffffffL));
 					h.slices += n / 4;
 				}
+			}
 		}
 	}
 }

@@ -131,3 +131,20 @@ def test_autotune_times_the_untuned_layout(stub, na, fmt):
     assert layout(h) == want
     assert layout(plan(geom(256, 256, 128, 512, 384, 0.5, 0.5, 0.8, 0.8), {na}, {fmt})) == want
     """)
+
+
+def test_plan_creation_time_does_not_grow_with_slices(stub):
+    """The default launch shape comes from a bounded sample of z-groups: a plan
+    of 65535 slices takes no more than a few times a plan of 512 (over all groups
+    it takes about 60 times as long)."""
+    _run(stub, """
+    def best(nz):
+        t = []
+        for _ in range(7):
+            t0 = time.perf_counter()
+            h = plan(geom(128, 128, nz, 64, 400, 4.0, 240.0 / nz, 4.0, 4.0))
+            t.append(time.perf_counter() - t0)
+            lib.fdkhip_plan_destroy(h)
+        return min(t)
+    assert best(65535) < 5 * best(512), (best(65535), best(512))
+    """)
