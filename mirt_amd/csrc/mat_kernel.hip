@@ -79,13 +79,18 @@ __device__ __forceinline__ double mat_sample(const double *p, long i)
 // remainder a - q b is exact in one FMA and RN(q + r rh) is the correctly
 // rounded quotient (Markstein, "Computation of elementary functions on the IBM
 // RISC System/6000 processor", IBM J. Res. Dev. 34(1), 1990, theorem 8.2).
-// Needs a finite, |b| within [1e-60, 1e60] and no over- or underflow on the
-// way (|a| = 0 or above 2^-900); the callers see to it.
+// Needs |b| within [1e-60, 1e60] and no over- or underflow on the way: a NaN
+// comes of an overflow, and |a| is 0 or at least DIV_MIN, where the quotient is
+// above 2^-1000 and the remainder above 2^-910.  The kernel does workgroups
+// again that see another dividend of the weight (tprime, the other dividend,
+// may be smaller: bt = tprime / dt + wt is then wt).
 __device__ __forceinline__ double const_div(double a, double b, double rh, double rl)
 {
 	const double q = fma(a, rh, a * rl);
 	return fma(fma(-q, b, a), rh, q);
 }
+
+constexpr double DIV_MIN = 1e-240;   // above 2^-800
 
 __device__ __forceinline__ bool mat_moderate(double x)
 {
@@ -117,7 +122,8 @@ static_assert(MAT_NW * MAT_ZC <= 128, "two words of slice flags");
 // FAST: quotients by const_div and both samples of a row in one load -- for
 // the last column, whose right neighbour is the zero column ns+1, the pair to
 // its left with the weights moved one sample over.  A FAST workgroup that
-// meets a geometry outside const_div's range, or ends with a NaN sum (an
+// meets a geometry or (FP64 views; FP32 samples are too large) a dividend
+// outside const_div's range, or ends with a NaN sum (an
 // infinite sample gives NaN in const_div and in a zero weight's product, where
 // the reference may have an infinity or a number), sets its entry of a.redo;
 // the other form, the reference's arithmetic to the letter, is launched after
@@ -305,9 +311,12 @@ __global__ void __launch_bounds__(64 * MAT_NW, FAST ? 4 : 2) mat_kernel(const Ma
 				const double p1 = wL * (double) u0[g].x + wR * (double) u0[g].y;
 				const double p2 = wL * (double) u1[g].x + wR * (double) u1[g].y;
 				double p0 = wd * p1 + wu * p2;
-				if (WGT == MW_DIV)
-					p0 = FAST ? const_div(p0 * dsd2, w, rh, rl) : p0 * dsd2 / w;
-				else if (WGT == MW_MUL)
+				if (WGT == MW_DIV) {
+					const double d = p0 * dsd2;
+					if (FAST && sizeof(TP) == 8)
+						bad = bad || (fabs(d) < DIV_MIN && d != 0.0);
+					p0 = FAST ? const_div(d, w, rh, rl) : d / w;
+				} else if (WGT == MW_MUL)
 					p0 = p0 * w;
 				acc[k] = acc[k] + p0;                // cbct_back.m:251
 			}

@@ -263,3 +263,44 @@ def test_mat_slice_groups(device, nz, ns, dt, dtype):
     beta = np.linspace(0, 6, 11)
     got = _host_call(g, proj, beta, scale=0.3)
     assert np.array_equal(got, O.back_mat_f64(g, proj, beta, scale=0.3))
+
+
+@pytest.mark.parametrize("size", [1.0, 1e-230, 1e-247, 1e-300, 1e-308, 1e-310, 1e-312, 1e295])
+def test_mat_arc_quotients_are_divisions(device, size):
+    """The arc's weight on FP64 views: bit for bit the division form, also for
+    samples so large or so small (denormal ones among them) that the reciprocal
+    quotient's remainder leaves the range, where about one quotient in a million
+    would be off by a unit.  The division form runs where a source height is
+    beyond 1e60, here that of a view of zeros, which adds nothing."""
+    g = O.geom((96, 90, 64), (1.1, -1.1, 0.7), (0.25, 0.0, -1.5), 541.0, 949.0, 0.0,
+               101, 33, (1.9, 2.3), (0.25, 0.5))
+    proj = np.random.default_rng(3).standard_normal((101, 33, 24)) * size
+    proj[:, :, 5] = 0.0
+    proj[::3, :, 7] = 0.0
+    beta, zs = np.linspace(0, 6, 24), np.zeros(24)
+    got = _host_call(g, proj, beta, zs=zs)
+    zs[5] = 1e61
+    want = _host_call(g, proj, beta, zs=zs)
+    assert np.any(want) and np.array_equal(got, want), np.count_nonzero(got != want)
+
+
+def test_mat_helix_slice_groups(device):
+    """cbct_back_helix's use_mex = 0 route over 140 slices: both words of a
+    workgroup's slice flags and a second workgroup of slices (the cases above
+    have 23 slices).  Flat detector, so bit for bit."""
+    from mirt_amd import cbct_back_helix, ct_geom, image_geom
+    from mirt_amd.cbct_back import _views
+    cg = ct_geom("fan", ns=40, nt=12, na=150, ds=2.0, dt=2.2, dsd=949.0, dso=541.0,
+                 dfs=np.inf, orbit=1800, pitch=1.0, source_z0="center")
+    ig = image_geom(nx=10, ny=9, nz=140, dx=3.0, dz=0.55)
+    g = O.geom((ig.nx, ig.ny, ig.nz), (ig.dx, ig.dy, ig.dz), (0, 0, 0), cg.dso, cg.dsd, cg.dfs,
+               cg.ns, cg.nt, (cg.ds, cg.dt), (0, 0))
+    proj = np.asfortranarray(np.random.default_rng(6).standard_normal((40, 12, 150))
+                             .astype(np.float32))
+    with pytest.warns(UserWarning, match="always extrapolates"):
+        got = cbct_back_helix(proj, cg, ig, use_mex=0)
+    first, last, sc = O.helix_mat_slices(g, cg.na, cg.orbit, cg.pitch, cg.source_zs, 1)
+    want = O.back_helix_mat_f64(g, proj, _views(cg, cg.na), cg.source_zs, first, last,
+                                mask=ig.mask_or, slice_scale=sc)
+    for part in (slice(0, 64), slice(64, 128), slice(128, 140)):
+        assert np.any(want[:, :, part]) and np.array_equal(got[:, :, part], want[:, :, part]), part
