@@ -359,7 +359,8 @@ int fdkhip_batch_create(fdkhip_batch **batch, int32_t nscan,
 /* proj[i], scale[i] (F16/BF16 only; scale may be NULL for F32) and image[i]
  * are scan i's device buffers as in fdkhip_plan_execute.  Asynchronous on
  * `stream`; replayed from a HIP graph from the second call with the same
- * pointers on. */
+ * pointers on.  On a stream that the caller captures, one launch per scan goes
+ * into the caller's graph. */
 int fdkhip_batch_execute(fdkhip_batch *batch, const void *const *proj,
 	const float *const *scale, float *const *image, void *stream);
 

@@ -2728,15 +2728,15 @@ static long long plan_work(const fdkhip_plan *p)
 	return (long long) p->na * p->geom.nx * p->geom.ny * (p->zs_hi - p->zs_lo);
 }
 
-// the backprojection alone on the uploaded arguments: the persistent kernel
-// (with its queue reset), or each scan's own launch.  The per-scan launches
+// the backprojection alone: the persistent kernel on the uploaded arguments
+// (with its queue reset), or each scan's own launch on host_args.  The per-scan launches
 // go to two streams, `s` and the batch's side stream (forked from `s` and
 // joined back into it), the scans in descending order of size (plan_work)
 // each to the stream with less queued: the next scan's workgroups then
 // fill the CUs that a launch's last round leaves idle.
-static int batch_kernel_launch(fdkhip_batch *b, hipStream_t s)
+static int batch_kernel_launch(fdkhip_batch *b, bool per_scan, hipStream_t s)
 {
-	if (b->per_scan) {
+	if (per_scan) {
 		if (!b->side) {
 			HIP_TRY(hipStreamCreateWithFlags(&b->side, hipStreamNonBlocking));
 			HIP_TRY(hipEventCreateWithFlags(&b->fork_ev, hipEventDisableTiming));
@@ -2778,7 +2778,7 @@ static int batch_kernel_launch(fdkhip_batch *b, hipStream_t s)
 // Per-scan zero fills and padded copies, then the backprojection
 // (batch_kernel_launch).  With `ev`, ev[0..2] are recorded before the
 // per-scan steps, between them and the backprojection, and after it.
-static int batch_launch(fdkhip_batch *b, const void *const *proj, const float *const *scale,
+static int batch_launch(fdkhip_batch *b, bool per_scan, const void *const *proj,
 	float *const *image, hipStream_t s, hipEvent_t *ev = nullptr)
 {
 	if (ev)
@@ -2797,7 +2797,7 @@ static int batch_launch(fdkhip_batch *b, const void *const *proj, const float *c
 	}
 	if (ev)
 		HIP_TRY(hipEventRecord(ev[1], s));
-	int rc = batch_kernel_launch(b, s);
+	int rc = batch_kernel_launch(b, per_scan, s);
 	if (rc)
 		return rc;
 	if (ev)
@@ -2820,9 +2820,9 @@ static int batch_check(fdkhip_batch *b, const void *const *proj, const float *co
 	return FDKHIP_OK;
 }
 
-// per-scan kernel arguments for these buffers -> device (ordered on `s`)
-static int batch_upload_args(fdkhip_batch *b, const void *const *proj,
-	const float *const *scale, float *const *image, hipStream_t s, int na_cap = 0)
+// per-scan kernel arguments for these buffers
+static void batch_make_args(fdkhip_batch *b, const void *const *proj,
+	const float *const *scale, float *const *image, int na_cap = 0)
 {
 	b->host_args.resize(b->nscan);
 	for (int i = 0; i < b->nscan; ++i) {
@@ -2830,12 +2830,38 @@ static int batch_upload_args(fdkhip_batch *b, const void *const *proj,
 		if (na_cap > 0)
 			b->host_args[i].g.na = std::min(b->host_args[i].g.na, na_cap);
 	}
+}
+
+// ... and, for the persistent kernel, -> device (ordered on `s`)
+static int batch_upload_args(fdkhip_batch *b, const void *const *proj,
+	const float *const *scale, float *const *image, hipStream_t s, int na_cap = 0)
+{
+	batch_make_args(b, proj, scale, image, na_cap);
 	if (b->per_scan)
 		return FDKHIP_OK;   // each launch takes its arguments by value
 	HIP_TRY(hipMemcpyAsync(b->d_scans, b->host_args.data(), sizeof(BackArgs) * b->nscan,
 		hipMemcpyHostToDevice, s));
 	HIP_TRY(hipStreamSynchronize(s));   // host_args may be rewritten by the next call
 	return FDKHIP_OK;
+}
+
+// Whether the caller captures `s`.
+static bool is_capturing(hipStream_t s)
+{
+	hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+	if (hipStreamIsCapturing(s, &st) != hipSuccess)
+		(void) hipGetLastError();   // the null stream beside a capture: the launch will say so
+	return st == hipStreamCaptureStatusActive;
+}
+
+// Into a caller's graph: one launch per scan in either form (the same bits), since
+// those take their arguments by value, where the persistent kernel's are on the
+// device and change with the next call's buffers; and nothing that waits.
+static int batch_capture(fdkhip_batch *b, const void *const *proj, const float *const *scale,
+	float *const *image, hipStream_t s)
+{
+	batch_make_args(b, proj, scale, image);
+	return batch_launch(b, true, proj, image, s);
 }
 
 extern "C" int fdkhip_batch_execute_direct(fdkhip_batch *b, const void *const *proj,
@@ -2845,18 +2871,20 @@ extern "C" int fdkhip_batch_execute_direct(fdkhip_batch *b, const void *const *p
 	if (rc)
 		return rc;
 	hipStream_t s = (hipStream_t) stream;
+	if (is_capturing(s))
+		return batch_capture(b, proj, scale, image, s);
 	rc = batch_upload_args(b, proj, scale, image, s);
 	if (rc)
 		return rc;
 	batch_drop_graph(b);   // the uploaded arguments may differ from the graph's
-	return batch_launch(b, proj, scale, image, s);
+	return batch_launch(b, b->per_scan, proj, image, s);
 }
 
 // A second call with the buffers of the one before captures the launches and
 // replays them from then on; any other call launches directly, since a graph
 // for buffers that do not come back costs its capture and instantiation and
-// saves nothing.
-
+// saves nothing.  (A graph launched on a capturing stream would run at once and
+// not be in the caller's graph.)
 extern "C" int fdkhip_batch_execute(fdkhip_batch *b, const void *const *proj,
 	const float *const *scale, float *const *image, void *stream)
 {
@@ -2864,6 +2892,8 @@ extern "C" int fdkhip_batch_execute(fdkhip_batch *b, const void *const *proj,
 	if (rc)
 		return rc;
 	hipStream_t s = (hipStream_t) stream;
+	if (is_capturing(s))
+		return batch_capture(b, proj, scale, image, s);
 	bool same = (int) b->g_proj.size() == b->nscan;
 	for (int i = 0; same && i < b->nscan; ++i)
 		same = b->g_proj[i] == proj[i] && b->g_image[i] == image[i]
@@ -2882,8 +2912,9 @@ extern "C" int fdkhip_batch_execute(fdkhip_batch *b, const void *const *proj,
 	if (!b->gexec) {
 		if (!b->cap_stream)
 			HIP_TRY(hipStreamCreateWithFlags(&b->cap_stream, hipStreamNonBlocking));
+		batch_make_args(b, proj, scale, image);   // a caller's capture may have changed them
 		HIP_TRY(hipStreamBeginCapture(b->cap_stream, hipStreamCaptureModeThreadLocal));
-		rc = batch_launch(b, proj, scale, image, b->cap_stream);
+		rc = batch_launch(b, b->per_scan, proj, image, b->cap_stream);
 		hipGraph_t graph = nullptr;
 		hipError_t e = hipStreamEndCapture(b->cap_stream, &graph);
 		b->graph = graph;
@@ -2916,7 +2947,7 @@ extern "C" int fdkhip_batch_autotune(fdkhip_batch *b, const void *const *proj,
 	// the first kTuneViews views of every scan
 	rc = batch_upload_args(b, proj, scale, image, s);
 	if (!rc)
-		rc = batch_launch(b, proj, scale, image, s);
+		rc = batch_launch(b, b->per_scan, proj, image, s);
 	if (rc)
 		return rc;
 	// per shape: the chosen per-scan heights, then (where that choice moved
@@ -2944,7 +2975,7 @@ extern "C" int fdkhip_batch_autotune(fdkhip_batch *b, const void *const *proj,
 					return rc;
 				float t = 0.f;
 				rc = time_launches([&](hipStream_t st) {
-					return batch_kernel_launch(b, st);
+					return batch_kernel_launch(b, b->per_scan, st);
 				}, s, reps, &t);
 				if (rc)
 					return rc;
@@ -2971,7 +3002,7 @@ extern "C" int fdkhip_batch_autotune(fdkhip_batch *b, const void *const *proj,
 		return rc;
 	float t_scan = 0.f;
 	rc = time_launches([&](hipStream_t st) {
-		return batch_kernel_launch(b, st);
+		return batch_kernel_launch(b, b->per_scan, st);
 	}, s, reps, &t_scan);
 	if (rc)
 		return rc;
@@ -3010,7 +3041,7 @@ extern "C" int fdkhip_batch_profile(fdkhip_batch *b, const void *const *proj,
 		}
 	double sum[2] = {0, 0};
 	for (int r = 0; r < reps && !rc; ++r) {
-		rc = batch_launch(b, proj, scale, image, s, ev);
+		rc = batch_launch(b, b->per_scan, proj, image, s, ev);
 		if (!rc && hipEventSynchronize(ev[2]) != hipSuccess)
 			rc = fail(FDKHIP_EHIP, "hipEventSynchronize");
 		for (int k = 0; k < 2 && !rc; ++k) {

@@ -292,3 +292,37 @@ def test_batch_argument_errors(device):
     b16 = _batch(cases, fmt="f16", math_mode="fast")
     with pytest.raises(ValueError):
         b16([p.half() for p in projs])   # no scales
+
+
+@pytest.mark.parametrize("warm", [0, 1, 3])
+@pytest.mark.parametrize("per_scan", [False, True])
+def test_batch_in_a_callers_graph(device, per_scan, warm):
+    """A batch captured by the caller, without and after calls on the same
+    buffers: every replay computes the images of the data then in the buffers,
+    whatever the batch ran on other buffers in between."""
+    import torch
+    cases = _cases()
+    b = _batch(cases)
+    b.set_per_scan() if per_scan else b.set_config(8, 16)
+    projs = [torch.from_numpy(p).to(device) for _, p, _, _ in cases]
+    outs = [torch.empty((g.ny, g.nx, g.nz), device=device) for g, _, _, _ in cases]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    for _ in range(warm):
+        b(projs, outs=outs, stream=side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        b(projs, outs=outs)
+    for rep in range(3):
+        new = [np.random.default_rng(rep).standard_normal(p.shape, dtype=np.float32)
+               for _, p, _, _ in cases]
+        for t, o, x in zip(projs, outs, new):
+            t.copy_(torch.from_numpy(x))
+            o.fill_(float("nan"))
+        b([p.clone() for p in projs])
+        graph.replay()
+        torch.cuda.synchronize()
+        for i, (g, _, beta, mask) in enumerate(cases):
+            assert np.array_equal(outs[i].cpu().numpy(), O.back_ts_f32(g, new[i], beta, mask)), \
+                (rep, i)

@@ -148,3 +148,34 @@ def test_plan_creation_time_does_not_grow_with_slices(stub):
         return min(t)
     assert best(65535) < 5 * best(512), (best(65535), best(512))
     """)
+
+
+@pytest.mark.parametrize("per_scan", [False, True])
+def test_batch_into_a_callers_graph(stub, per_scan):
+    """A batch on a stream that the caller captures launches every scan on it, and
+    neither copies, waits, nor launches a graph of its own (which would run at once,
+    outside the capture), whatever calls came before; those after it go on as if it
+    had not been."""
+    _run(stub, f"""
+    n, per_scan = 3, {per_scan}
+    garr = (_lib.Geom * n)(*[geom(32 + 8 * i, 32, 24, 64, 48, 2.0, 2.0, 4.0, 4.0) for i in range(n)])
+    beta = np.linspace(0, 6, 20)
+    b, ba = C.c_void_p(), (C.c_void_p * n)(*[beta.ctypes.data] * n)
+    _lib.check(lib.fdkhip_batch_create(C.byref(b), n, garr, (C.c_int32 * n)(20, 20, 20), ba, None, F32, 0))
+    _lib.check(lib.fdkhip_batch_set_per_scan(b) if per_scan else lib.fdkhip_batch_set_config(b, 8, 16, 0))
+    bufs = [(C.c_void_p * n)(*[(k + i) << 20 for i in range(n)]) for k in (1, 8)]
+    S = C.c_void_p(77)
+    def execute(k, direct=False):
+        fake.fake_clear()
+        f = lib.fdkhip_batch_execute_direct if direct else lib.fdkhip_batch_execute
+        _lib.check(f(b, bufs[k], None, bufs[k], S))
+        return [r[0] for r in log()]
+    for warm in range(4):
+        fake.fake_capturing(1)
+        for k, direct in ((0, False), (1, False), (0, True), (1, True)):
+            kinds = execute(k, direct)
+            assert set(kinds) == {{"launch"}} and len(kinds) >= 2 * n, (warm, kinds)
+        fake.fake_capturing(0)
+        kinds = execute(0)
+        assert ("graphlaunch" in kinds) == (warm > 0), (warm, kinds)
+    """)
