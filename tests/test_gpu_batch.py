@@ -326,3 +326,41 @@ def test_batch_in_a_callers_graph(device, per_scan, warm):
         for i, (g, _, beta, mask) in enumerate(cases):
             assert np.array_equal(outs[i].cpu().numpy(), O.back_ts_f32(g, new[i], beta, mask)), \
                 (rep, i)
+
+
+@pytest.mark.parametrize("fmt", ["f32", "f16"])
+@pytest.mark.parametrize("per_scan", [False, True])
+def test_batch_graph_replays(device, per_scan, fmt):
+    """Five calls on the same buffers, new data before each and nothing else in
+    between (a direct launch, the capture, three replays): each gives the images
+    that another batch, which never repeats a buffer, gives for its data."""
+    import torch
+    from mirt_amd import quantize_views
+    cases = _cases() + [_off_fov_case()]
+    b, ref = _batch(cases, fmt), _batch(cases, fmt)
+    for x in (b, ref):
+        x.set_per_scan() if per_scan else x.set_config(8, 16)
+        assert x.per_scan == per_scan
+    new = lambda rep: [quantize_views(torch.from_numpy(np.random.default_rng(rep).standard_normal(  # noqa: E731
+        p.shape, dtype=np.float32)).to(device), fmt) if fmt != "f32" else (torch.from_numpy(
+            np.random.default_rng(rep).standard_normal(p.shape, dtype=np.float32)).to(device), None)
+        for _, p, _, _ in cases]
+    bufs = new(99)
+    scales = None if fmt == "f32" else [s for _, s in bufs]
+    outs = [torch.empty((g.ny, g.nx, g.nz), device=device) for g, _, _, _ in cases]
+    for rep in range(5):
+        data = new(rep)
+        for (q, s), (x, y), o in zip(bufs, data, outs):
+            q.copy_(x)
+            if s is not None:
+                s.copy_(y)
+            o.fill_(float("nan"))
+        b([q for q, _ in bufs], scales, outs)
+        torch.cuda.synchronize()
+        want = ref([x for x, _ in data], None if fmt == "f32" else [y for _, y in data],
+                   graph=False)
+        for i, (g, _, beta, mask) in enumerate(cases):
+            assert torch.equal(outs[i], want[i]), (rep, i)
+            if fmt == "f32":
+                assert np.array_equal(outs[i].cpu().numpy(),
+                                      O.back_ts_f32(g, data[i][0].cpu().numpy(), beta, mask)), (rep, i)

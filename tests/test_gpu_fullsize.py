@@ -283,3 +283,36 @@ def test_fullsize_helix(device):
         err = O.rel_l2(got, want)
         print(f"clinical_helix {fmt} vs FP32 EXACT: relL2 {err:.2e}", flush=True)
         assert err <= bar, (fmt, err)
+
+
+def test_fullsize_uneven_batch_persistent(device):
+    """All 32 uneven scans in the persistent kernel, whose form has to be asked
+    for at these sizes: sampled columns of every scan bit for bit equal to the
+    oracle over a direct launch, the graph's first launch and a replay, each with
+    new data."""
+    import torch
+    from mirt_amd import FdkBatch, geom_of
+    from mirt_amd.cbct_back import _views
+    from mirt_amd.workloads import uneven_scans
+    scans = uneven_scans(32)
+    betas = [_views(s.cg, s.cg.na) for s in scans]
+    batch = FdkBatch([(geom_of(s.cg, s.ig), b, None) for s, b in zip(scans, betas)])
+    assert batch.per_scan                      # scans of 128 and more workgroups
+    batch.set_config(8, 16)
+    assert not batch.per_scan and len(set(batch.scan_zper)) > 1
+    projs = [_noise_views(s.cg, device, seed=0) for s in scans]
+    outs = [torch.empty((s.ig.ny, s.ig.nx, s.ig.nz), device=device) for s in scans]
+    for rep in range(3):
+        for i, p in enumerate(projs):
+            p.copy_(_noise_views(scans[i].cg, device, seed=100 * rep + i))
+            outs[i].fill_(float("nan"))
+        batch(projs, outs=outs)
+        torch.cuda.synchronize()
+        for i, s in enumerate(scans):
+            cols = _cols(s.ig, 8, seed=10 * rep + i)
+            mask = np.ones((s.ig.ny, s.ig.nx), np.uint8)
+            want = O.back_ts_f32(_oracle_geom(s.cg, s.ig), projs[i].cpu().numpy(), betas[i], mask,
+                                 cols=cols)
+            got = outs[i].cpu().numpy().reshape(-1, s.ig.nz)[cols]
+            assert np.array_equal(got, want), (rep, i, O.rel_l2(got, want))
+        print(f"persistent batch rep {rep}", flush=True)

@@ -179,3 +179,23 @@ def test_batch_into_a_callers_graph(stub, per_scan):
         kinds = execute(0)
         assert ("graphlaunch" in kinds) == (warm > 0), (warm, kinds)
     """)
+
+
+@pytest.mark.parametrize("ny,per_scan", [(120, False), (128, True)])
+def test_batch_default_form(stub, ny, per_scan):
+    """A new batch takes one launch per scan from 128 workgroups a scan in the mean
+    on (64 x ny columns, one z-group: ny workgroups; one scan of 64 more and one of
+    64 fewer), the work queue below."""
+    _run(stub, f"""
+    ys = ({ny}, {ny} + 64, {ny} - 64)
+    garr = (_lib.Geom * 3)(*[geom(64, y, 16, 64, 48, 2.0, 2.0, 4.0, 4.0) for y in ys])
+    beta = np.linspace(0, 6, 20)
+    b, ba = C.c_void_p(), (C.c_void_p * 3)(*[beta.ctypes.data] * 3)
+    for fmt in (F32, F16):
+        _lib.check(lib.fdkhip_batch_create(C.byref(b), 3, garr, (C.c_int32 * 3)(20, 20, 20), ba, None,
+                                           fmt, 0))
+        cfg = (C.c_int32 * 6)()
+        _lib.check(lib.fdkhip_batch_config(b, cfg))
+        assert (cfg[0] == 0) == {per_scan} and cfg[5] == 3 * {ny}, list(cfg)
+        lib.fdkhip_batch_destroy(b)
+    """)
