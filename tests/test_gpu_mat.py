@@ -304,3 +304,49 @@ def test_mat_helix_slice_groups(device):
                                 mask=ig.mask_or, slice_scale=sc)
     for part in (slice(0, 64), slice(64, 128), slice(128, 140)):
         assert np.any(want[:, :, part]) and np.array_equal(got[:, :, part], want[:, :, part]), part
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("ns,nt,dfs", [(1 << 24, 2, np.inf), ((1 << 24) - 1, 2, np.inf),
+                                       (2, 1 << 24, np.inf), (2, 1 << 24, 0.0)])
+def test_mat_long_detector_side(device, ns, nt, dfs, dtype):
+    """Detector sides of 2^24 samples, whose offsets are 64 bits wide, and one
+    below, the largest with 32-bit offsets of 24-bit factors.  (No arc of 2^24
+    columns: a last place of its atan2 is 1e-9 of a column there.)"""
+    ds, dt = (2e-5, 60.0) if ns > nt else (90.0, 1e-5)
+    g = O.geom((9, 10, 18), (11.0, -11.0, 3.0), (0.25, 0.0, -1.5), 541.0, 949.0, dfs,
+               ns, nt, (ds, dt), (0.25, 0.5))
+    proj = np.random.default_rng(ns % 1000).standard_normal((2, nt, ns)).astype(dtype)
+    proj, beta = proj.transpose(2, 1, 0), np.array([0.3, 2.0])
+    want = O.back_mat_f64(g, proj, beta)
+    assert np.any(want)
+    _compare("arc" if dfs == 0 else "flat", _host_call(g, proj, beta), want)
+
+
+@pytest.mark.parametrize("dtype,ns", [("float32", 32768), ("float64", 16384)])
+def test_mat_view_over_4gib(device, dtype, ns):
+    """One parallel view of more than 4 GiB, its last rows beyond the reach of
+    32-bit byte offsets: bit for bit what those rows alone give on a detector of
+    64 rows (positions and weights are exact in binary on both)."""
+    import torch
+    from mirt_amd import _lib
+    lib = _lib.load()
+    nt, rows = 32800, 64
+    big = torch.empty((1, nt, ns), dtype=getattr(torch, dtype), device=device)
+    assert big.numel() * big.element_size() > 1 << 32
+    big[:, -rows:] = torch.randn((1, rows, ns), dtype=big.dtype, device=device)
+    shape = dict(nxyz=(30, 3, 18), dxyz=(512.25, -1.0, 3.25), cxyz=(0, 0, 0), dso=np.inf,
+                 dsd=np.inf, dfs=np.inf, ns=ns, dst=(1.0, 1.0))
+    # wt = (nt + 1) / 2 + offset: 30.5 rows from the end on both detectors
+    g = O.geom(nt=nt, ost=(0.25, (nt - 1) / 2 - 30.5), **shape)
+    small = O.geom(nt=rows, ost=(0.25, (rows - 1) / 2 - 30.5), **shape)
+    beta = np.zeros(1)
+    img = torch.empty((18, 3, 30), dtype=torch.float64, device=device)
+    _lib.check(lib.fdkhip_cbct_back_mat_direct(
+        C.byref(_geom(g)), C.c_void_p(big.data_ptr()), int(dtype == "float64"), 1,
+        C.c_void_p(beta.ctypes.data), None, 1, 0.0, None, 1.0, C.c_void_p(img.data_ptr()),
+        C.c_void_p(torch.cuda.current_stream().cuda_stream), None))
+    tail = big[:, -rows:].cpu().numpy().transpose(2, 1, 0)
+    want = O.back_mat_f64(small, tail, beta)
+    got = img.cpu().numpy().transpose(2, 1, 0)
+    assert np.any(want) and np.array_equal(got, want), float(np.abs(got - want).max())
