@@ -92,18 +92,20 @@ struct ViewGeo {
 };
 
 // DIRECT (FP16/BF16) modes: the z coordinate at which each column's record holds
-// u.  On an axial scan it is the half slice nearest to the source's plane: u is
-// wt + 1 in that plane, so it takes no rounding of the column's own where the
-// plane is at a half slice and one elsewhere; distances from it are exact, and a
-// slice's u has the roundings of its own two fused multiply-adds, the same
-// whatever the z-group's height: a launch's shape does not change its results.
-// (512 rows, 128 slices that reach at most both ends of the detector, emulated in
-// FP32: rms error of u 0.95e-5 rows; 1.2e-5 from the z-group's first slice, 1.4e-5
-// from the slice next to the source's plane with u carried there from the cone's
-// lower edge.)  On a helix, whose source plane moves, the z-group's first slice.
+// u.  On an axial scan it is the source's plane, where u is wt + 1 for every column:
+// no rounding of the column's own; a slice's distance from the plane is one
+// subtraction (exact where wz is a half slice, and otherwise while the distance is
+// below the power of two above wz), and its u has the roundings of its own two fused
+// multiply-adds, the same whatever the z-group's height: a launch's shape does not
+// change its results.
+// (512 rows, emulated in FP32, rms error of u in 1e-5 rows, from here / from the half
+// slice nearest to the plane / from the z-group's first slice: 128 slices that reach at
+// most both ends of the detector 0.95 / 0.95 / 1.2; 256 slices of 1.2 mm, 33.33 slices
+// off centre 0.86 / 1.24 / 0.95.)  On a helix, whose source plane moves, the z-group's
+// first slice.
 __device__ __forceinline__ float anchor_z(const GeomF &g, bool axial, int zg0)
 {
-	return axial ? 0.5f * rintf(2.f * g.wz) : (float) zg0;
+	return axial ? g.wz : (float) zg0;
 }
 
 // Entry of a table that no kernel writes while it is read, at an index that is
@@ -321,8 +323,7 @@ __device__ __forceinline__ bool setup_walk(const GeomF &g, const ColSetup &c,
 // Slice range of one z-group for the FP16/BF16 paths, in u = t_bin + 1 (the
 // padded detector row coordinate, > 0 for every slice that reads a sample).
 // u is evaluated in closed form, as the consumer evaluates it:
-//   U0 = wt + 1 + (anchor_z - wz) * t_inc, or on a helix
-//        u(iz_min) + (zg0 - iz_min) * t_inc
+//   U0 = wt + 1, or on a helix u(iz_min) + (zg0 - iz_min) * t_inc
 //   U8 = U0 + (z8 - anchor_z) * t_inc            (every eighth slice of the group)
 //   u  = U8 + j * t_inc                          (slice z8 + j)
 // each step one fmaf (one rounding each; nearer the exact value than the
@@ -340,7 +341,7 @@ __device__ __forceinline__ bool setup_direct(const GeomF &g, const ColSetup &c, 
 {
 	const float ti = c.t_inc;
 	const float za = anchor_z(g, vg.axial, zg0);
-	const float U0 = vg.axial ? fmaf(za - g.wz, ti, g.wt + 1.f)
+	const float U0 = vg.axial ? g.wt + 1.f
 		: fmaf((float) (zg0 - c.iz_min), ti, c.t_bin + 1.f);
 	Uk[0] = U0;
 	auto uz = [&](int z) {           // z in [zg0, zg1)
@@ -1034,7 +1035,7 @@ __device__ __forceinline__ int2 view_window(const BackArgs &a, int v)
 template <int NCW, int R, int ZL, int FMT, bool WINDOW>
 __device__ __forceinline__ int consume_direct(const BackArgs &a, int bo,
 	const Lds<NCW * R, false> &L, int v0, int v, int nv, int wave, int lane, int zg0,
-	float (&accs)[R][ZL])
+	const float (&dz)[R][ZL / 8], float (&accs)[R][ZL])
 {
 	const GeomF &g = a.g;
 	// the lane's record addresses are made anew for each run: kept over the stages
@@ -1044,15 +1045,11 @@ __device__ __forceinline__ int consume_direct(const BackArgs &a, int bo,
 	const float4 *P4 = reinterpret_cast<const float4 *>(fdk_lds + bo + L.P) + lane;
 	const float2 *Q2 = reinterpret_cast<const float2 *>(fdk_lds + bo + L.Q) + lane;
 	const int *ZR = reinterpret_cast<const int *>(fdk_lds + bo + L.vinfo);
-	const float za = anchor_z(g, !WINDOW, zg0);
 	// relative to the z-group: chunk r starts at slice zoff(r)
 	auto zoff = [&](int r) { return (wave + r * NCW) * ZL; };
 	// U8: one fused multiply-add from the anchor for every eight slices, whatever
 	// the launch shape
-	const float zf = (float) (zg0 + zoff(0)) - za;
-	auto u8 = [&](int r, int j, float ti, float U0) {
-		return fmaf(zf + (float) (r * NCW * ZL + (j & ~7)), ti, U0);
-	};
+	auto u8 = [&](int r, int j, float ti, float U0) { return fmaf(dz[r][j >> 3], ti, U0); };
 	// window of chunk r relative to its first slice, clamped to [0, ZL]
 	auto window = [&](int2 wa, int r) {
 		const int zc = zg0 + zoff(r);
@@ -1294,6 +1291,15 @@ __device__ __forceinline__ void tile_pipeline(const BackArgs &a, int tile, int g
 #pragma unroll
 			for (int j = 0; j < ZL; ++j)
 				accs[r][j] = 0.f;
+		// distance of every eighth slice from the anchor (the same in every lane: kept in
+		// scalar registers)
+		float dz[R][ZL / 8];
+#pragma unroll
+		for (int r = 0; r < R; ++r)
+#pragma unroll
+			for (int k = 0; k < ZL / 8; ++k)
+				dz[r][k] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(
+					(float) (zg0 + (wave + r * NW) * ZL + 8 * k) - anchor_z(g, !WIN, zg0))));
 		__syncthreads();
 		for (int s = 0, v = 0; s < nstage;) {   // v: the stage's next view
 			const int v0 = va + s * a.vstage, nv = min(a.vstage, vb - v0);
@@ -1305,7 +1311,7 @@ __device__ __forceinline__ void tile_pipeline(const BackArgs &a, int tile, int g
 				// chunks wave + r NW of the z-group in one pass over the
 				// stage's views (u is in closed form from the group's U0)
 				v = consume_direct<NW, R, ZL, FMT, WIN>(a, (s & 1) * L.total, L, v0, v, nv, wave,
-					lane, zg0, accs);
+					lane, zg0, dz, accs);
 			}
 			if (v == nv) {
 				__syncthreads();

@@ -280,6 +280,36 @@ def test_16bit_row_coordinate_rounding(device, dz, fmt):
 
 
 @pytest.mark.parametrize("fmt", ["f16", "bf16"])
+@pytest.mark.parametrize("dz,offset", [(0.7, 72.8), (1.2, 72.8), (1.2, 0.3), (1.3, -0.45),
+                                       (0.9, -40.7)])
+def test_16bit_row_coordinate_rounding_off_centre(device, dz, offset, fmt):
+    """As above where the source's plane is not at a half slice: the plane itself
+    brings no rounding of the row, a slice's distance from it at most one (none
+    where the difference is a float)."""
+    import torch
+    nt, nz = 512, 256
+    g = O.geom((8, 8, nz), (1.0, -1.0, dz), (0, 0, offset), np.inf, np.inf, 0.0,
+               16, nt, (1.0, 1.0), (0.0, 0.0))
+    dtype = {"f16": torch.float16, "bf16": torch.bfloat16}[fmt]
+    sign = (1.0 - 2.0 * (np.arange(nt) % 2)).astype(np.float32)
+    q = torch.from_numpy(np.broadcast_to(sign, (1, 16, nt)).copy()).to(device, dtype)
+    img = _plan(g, np.zeros(1), np.ones((8, 8), np.uint8), fmt)(
+        q, torch.ones(1, device=device)).cpu().numpy()
+    ti = float(np.float32(dz))
+    wz = float(np.float32((nz - 1) / 2 + float(np.float32(offset))))
+    z = np.arange(nz)
+    u, u8 = (nt / 2 + 0.5 + (zz - wz) * ti for zz in (z, z & ~7))
+    inside = (u > 1) & (u < nt) & (u8 > 1)
+    assert inside.sum() > nz / 2
+    want = np.where(np.floor(u) % 2 == 1, 1.0, -1.0) * (1 - 2 * (u - np.floor(u)))
+    half = lambda x: np.spacing(x.astype(np.float32)).astype(np.float64) / 2      # noqa: E731
+    dist = (z & ~7) - wz
+    tol = 2 * (half(u8) + half(u) + np.abs(dist.astype(np.float32) - dist) * ti) + 2.0 ** -24
+    err = np.abs(img - want)
+    assert np.all((err <= tol)[..., inside]), (err / tol)[..., inside].max()
+
+
+@pytest.mark.parametrize("fmt", ["f16", "bf16"])
 @pytest.mark.parametrize("ds,ns", [(3.0, 40), (0.7, 180)])
 def test_16bit_bits_do_not_depend_on_slot(device, ds, ns, fmt):
     """Footprints of about 6 and 28 columns per 8 x 8 tile in slots that hold
