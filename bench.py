@@ -10,7 +10,7 @@ cosine weight and ramp filter.  The filtered views are stored on the device
 in FP16 with a per-view scale (FP32 and BF16 are timed beside it).
 
 One step = one backprojection of all views into the whole volume (the plan's
-graph: a zero fill of the slices no view reaches, the zero-padded copy of the
+launches: a zero fill of the slices no view reaches, the zero-padded copy of FP32
 views and the tiled kernel), projections and image resident in HBM.
 value = nx*ny*nz*na / t.  The roofline entry is for the backprojection kernel
 alone, timed with HIP events on its own stream (fdkhip_plan_profile).
@@ -568,8 +568,7 @@ def run_helix(args, dev):
     (clinical_helix: 3 turns of the clinical_arc detector) in native helical
     geometry: views [nt ns na] FP32 and the [nz nx ny] image resident on the
     device, a helical plan (fdkhip_plan_create_helix: the axial pipeline with
-    per-view source heights and slice windows, EXACT arithmetic), autotuned,
-    replayed from its HIP graph."""
+    per-view source heights and slice windows, EXACT arithmetic), autotuned."""
     import torch
     from mirt_amd import FdkPlan
     from mirt_amd.cbct_back import _views
@@ -824,7 +823,7 @@ def run_batch(args, dev, errors_without_baseline=False):
     U_eff = batch.count_updates()
     log(f"batch: {ms:.3f} ms/step, kernel {prof['back']:.3f} ms, {U / ms * 1e3:.3e} upd/s")
 
-    # the same scans one plan after another (each replayed from its graph)
+    # the same scans one plan after another
     ms_seq = None
     if not args.fmt_only:
         plans = [FdkPlan(geoms[i], betas[i], masks[i], fmt=fmt, math_mode=mm)

@@ -443,13 +443,15 @@ static void sample_heights(const fdkhip_plan *p, const double *beta, const uint8
 // few slices per wave.  The six costs (clocks) per arithmetic and what a view
 // gathered from memory costs were fitted to
 // the times of every shape, depth and residency for 39 scans (15 to 512 columns
-// a side, 14 to 256 slices, flat, arc and helical): the shape chosen is within
-// 4 % of the best one there in the mean.  Against 128-slice groups of 8 waves
-// for all (64-slice groups of 4 for short volumes):
+// a side, 14 to 256 slices, flat, arc and helical).  Over 40 others of that range
+// (profiles/default_launch_shape.md) the shape chosen takes 1.11 times the tuned
+// one's time in the geometric mean (median 1.03, largest 1.79), 128-slice groups of
+// 8 waves (64-slice groups of 4 for short volumes) 1.88 times in the mean, faster by
+// 12 % for one scan of the 40.  Against those fixed shapes:
 // 256 x 256 x 128 FP32 from 360 flat views of 512 x 384 2.0 ms for 2.9,
 // 256 x 256 x 192 FP32 helix of 1476 views 6.9 for 12.7,
 // 256 x 256 x 128 FP16 from 425 views of 713 x 477 2.6 for 6.6,
-// 64 x 64 x 32 FP32 from 64 views 0.050 for 0.081; never more than 6 % behind.
+// 64 x 64 x 32 FP32 from 64 views 0.050 for 0.081.
 struct ShapeCosts {
 	double wave, slice;            // issue per CU: per consumer wave, per slice of a column
 	double setup, words;           // producer: per view, per 64 footprint words
@@ -952,7 +954,9 @@ extern "C" int fdkhip_plan_execute_direct(fdkhip_plan *p, const void *proj,
 // At most three launches.  A graph of them belongs to one pair of buffers: a
 // caller with a new output per pass pays its capture, and a wait for the
 // device, each time (64 x 64 x 32 voxels, 64 FP32 views: 107 us a pass with
-// the graph, 82 launched directly).
+// the graph, 82 launched directly), and one whose buffers stay the same gains
+// nothing (us a pass replayed / direct: 16 x 16 x 8 voxels, 16 FP16 views 24.1 /
+// 16.4, 64 x 64 x 32, 64 FP32 views 86 / 81, 256 x 256 x 128, 360 views 2190 / 2203).
 extern "C" int fdkhip_plan_execute(fdkhip_plan *p, const void *proj, const float *scale,
 	float *image, void *stream)
 {
