@@ -441,13 +441,12 @@ static void sample_heights(const fdkhip_plan *p, const double *beta, const uint8
 // from the stage's LDS and the kernel's registers, so a taller z-group saves
 // set-up but costs residency by its larger footprints, and a short launch wants
 // few slices per wave.  The six costs (clocks) per arithmetic and what a view
-// gathered from memory costs were fitted to
-// the times of every shape, depth and residency for 39 scans (15 to 512 columns
-// a side, 14 to 256 slices, flat, arc and helical).  Over 40 others of that range
-// (profiles/default_launch_shape.md) the shape chosen takes 1.11 times the tuned
-// one's time in the geometric mean (median 1.03, largest 1.79), 128-slice groups of
-// 8 waves (64-slice groups of 4 for short volumes) 1.88 times in the mean, faster by
-// 12 % for one scan of the 40.  Against those fixed shapes:
+// gathered from memory costs were fitted to the times of every shape, depth and
+// residency for 39 scans (15 to 512 columns a side, 14 to 256 slices, flat, arc and
+// helical).  Over 40 others of that range the shape chosen takes 1.11 times the
+// tuned one's time in the geometric mean (median 1.03, largest 1.79), 128-slice
+// groups of 8 waves (64-slice groups of 4 for short volumes) 1.88 times in the mean,
+// faster by 12 % for one scan of the 40.  Against those fixed shapes:
 // 256 x 256 x 128 FP32 from 360 flat views of 512 x 384 2.0 ms for 2.9,
 // 256 x 256 x 192 FP32 helix of 1476 views 6.9 for 12.7,
 // 256 x 256 x 128 FP16 from 425 views of 713 x 477 2.6 for 6.6,
